@@ -243,16 +243,14 @@ void launch_split_rows(const MfmaBuffers &B, const uint16_t *x, uint32_t rows, u
  * starts of real checkpoint spans (about a quarter of the shipped tensors,
  * k3_rocm_ops.cu:207-223) take the MFMA kernels like aligned ones: the
  * 16-byte direct-to-LDS loads return the right bytes from 8-byte aligned
- * sources on gfx950 (measured, register and LDS forms). For the MFMA
- * kernels (all == 0) an expert with a tensor that is not even 8-byte
- * aligned gets no tiles, and B.unaligned hands it to the exact grouped
- * kernels. With all != 0 (the exact kernels' own tile list) every selected
- * expert gets tiles. */
+ * sources on gfx950 (measured, register and LDS forms). An expert with a
+ * tensor that is not even 8-byte aligned gets no tiles, and B.unaligned
+ * hands it to the exact kernels. */
 __global__ __launch_bounds__(1024) void tile_build_kernel(MfmaBuffers B,
                                                           const uint32_t *__restrict__ counts,
                                                           const uint32_t *__restrict__ offsets,
                                                           const k3_moe_expert *__restrict__ experts,
-                                                          uint32_t E, uint32_t all) {
+                                                          uint32_t E) {
     __shared__ uint32_t wave_tot[kTileClasses][16];
     __shared__ uint32_t odd_count;
     if (threadIdx.x == 0u) odd_count = 0u;
@@ -260,7 +258,7 @@ __global__ __launch_bounds__(1024) void tile_build_kernel(MfmaBuffers B,
     const uint32_t e = threadIdx.x, lane = e & 63u, wave = e >> 6;
     const uint32_t n = e < E ? counts[e] : 0u;
     bool odd = false;
-    if (n != 0u && !all) {
+    if (n != 0u) {
         const k3_moe_expert ex = experts[e];
         odd = (((uintptr_t)ex.gate_packed | (uintptr_t)ex.gate_scales | (uintptr_t)ex.down_packed |
                 (uintptr_t)ex.down_scales | (uintptr_t)ex.up_packed | (uintptr_t)ex.up_scales) %
@@ -1188,7 +1186,7 @@ bool launch_terms(const MfmaBuffers &B, uint16_t *y, const uint16_t *hidden,
     const uint32_t H = s.hidden, F = s.ffn;
     launch_split_rows<TERMS>(B, hidden, T, H, st);
     hipLaunchKernelGGL(tile_build_kernel, dim3(1), dim3(1024), 0, st, B, counts, offsets,
-                       experts, s.expert_count, 0u);
+                       experts, s.expert_count);
     mark(K3_MOE_STAGE_GATE_UP);
     GateUpArgs ga{B, nullptr, nullptr, token_index, experts, H, F, s.activation,
                   s.activation == 1u ? 1.0f : s.beta, s.activation == 1u ? 1.0f : s.linear_beta};
@@ -1246,14 +1244,6 @@ void mfma_tile_caps(uint32_t T, uint32_t k, uint32_t E, uint32_t caps[kTileClass
     caps[2] = upto(R / 65u);   /* 65-96 */
     /* > 96 rows: ceil(n / 128) <= n / 128 + 1 tiles each */
     caps[3] = (uint32_t)(R / 128u) + upto(R / 97u);
-}
-
-bool build_tiles_all(const MfmaBuffers &B, const uint32_t *counts, const uint32_t *offsets,
-                     const k3_moe_expert *experts, uint32_t E, hipStream_t st) {
-    if (E > 1024u) return false;
-    hipLaunchKernelGGL(tile_build_kernel, dim3(1), dim3(1024), 0, st, B, counts, offsets, experts,
-                       E, 1u);
-    return hipGetLastError() == hipSuccess;
 }
 
 bool mfma_supported(const k3_moe_shape &s) {

@@ -13,8 +13,8 @@
  *           grouped gate/up and down over the selected experts only (each
  *           expert's weights are read once per row block for all its
  *           tokens), then the slotted combine. K3_MOE_EXACT runs the w64
- *           VALU kernels below; K3_MOE_MFMA / _FP8 the scaled-MFMA tiles
- *           of k3_mfma.hip.
+ *           order on the fp32 matrix units (k3_exact.hip); K3_MOE_MFMA /
+ *           _FP8 the scaled-MFMA tiles of k3_mfma.hip.
  *
  * No host synchronisation anywhere: the expert ids never leave the device.
  * Every product uses the per-row w64 order of k3_ops.hip, so the decode and
@@ -23,6 +23,7 @@
 #include "k3_device.h"
 #include "k3_internal.h"
 #include "k3_decode.h"
+#include "k3_exact.h"
 #include "k3_mfma.h"
 #include "k3_topk.h"
 #include "../../include/k3_moe.h"
@@ -59,6 +60,7 @@ struct Workspace {
     k3_moe_expert *sel;
     uint16_t *y;
     MfmaBuffers mfma;
+    ExactGroup exact;
     size_t bytes;
 };
 
@@ -100,6 +102,7 @@ Workspace carve(void *base, const k3_moe_shape &s, uint32_t T) {
         /* MFMA path: activation codes reuse `act` (two byte planes of the
          * bf16 activation's size) */
         MfmaBuffers &m = w.mfma;
+        const size_t mfma_at = off;
         for (int t = 0; t < 2; t++) {
             m.xq[t] = take(1ull * T * s.hidden);
             m.xs[t] = take(1ull * T);
@@ -113,6 +116,22 @@ Workspace carve(void *base, const k3_moe_shape &s, uint32_t T) {
         m.tiles = (uint32_t *)take(12ull * ntiles);
         m.tile_count = (uint32_t *)take(4u * kTileClasses);
         m.unaligned = (uint32_t *)take(4ull * (s.expert_count + 1u));
+        /* exact path's tile lists: in place of the MFMA path's buffers, which
+         * hold at least 66 T + 12 tiles + 4 E bytes (F, H >= 32), i.e. the
+         * lists' 16 light + 16 heavy for every k <= 32 */
+        ExactGroup &x = w.exact;
+        x.lists = m.xq[0];
+        x.counts = w.counts;
+        x.offsets = w.offsets;
+        x.token_index = w.token_index;
+        x.route_index = w.route_index;
+        x.tokens = T;
+        x.routes = (uint32_t)routes;
+        x.E = s.expert_count;
+        x.H = s.hidden;
+        x.F = s.ffn;
+        const size_t lists = exact_list_bytes(x.routes, x.E);
+        if (off - mfma_at < lists) take(lists - (off - mfma_at));
     }
     w.bytes = off;
     return w;
@@ -267,213 +286,8 @@ bool launch_plan(uint32_t *counts, uint32_t *offsets, uint32_t *unique, uint32_t
 __device__ __forceinline__ float bf16_round(float v) { return bf16_to_f32(f32_to_bf16(v)); }
 
 /* ------------------------------------------------------------------------ */
-/* grouped (many tokens), exact order                                        */
+/* combine                                                                   */
 /* ------------------------------------------------------------------------ */
-
-/*
- * Work of a grouped exact workgroup: runs of plan rows [base, base + n) of
- * an expert e. Tile mode (list == nullptr): the tiles of the per-class
- * lists (at most 128 rows each, every selected expert; build_tiles_all),
- * walked with stride gridDim.y, so a heavy expert's rows spread over many
- * workgroups and no workgroup is launched past the tile count. List mode:
- * list = (count, expert ids), walked the same way, each expert's rows
- * whole (the MFMA path's fallback for experts whose tensors are not
- * 8-byte aligned).
- */
-struct ExactWork {
-    const uint32_t *tiles, *tile_count;
-    uint32_t cap[kTileClasses];
-    const uint32_t *list;       /* list mode: expert ids */
-    const uint32_t *list_count; /* their count */
-    const uint32_t *counts, *offsets;
-};
-
-/* Tile q of the tile lists (classes in order, tile_count[c] of class c
- * stored from the class's segment start); false past the last. */
-__device__ __forceinline__ bool exact_tile(const ExactWork &W, uint32_t q, uint32_t &e,
-                                           uint32_t &base, uint32_t &n) {
-    uint32_t first = 0u;
-#pragma unroll
-    for (int c = 0; c < kTileClasses; c++) {
-        const uint32_t tc = W.tile_count[c];
-        if (q < tc) {
-            const uint32_t *t = W.tiles + 3u * (first + q);
-            e = t[0];
-            base = t[1];
-            n = t[2];
-            return true;
-        }
-        q -= tc;
-        first += W.cap[c];
-    }
-    return false;
-}
-
-/* Gate/up of plan rows [base, base + n) of expert e, weight rows row0 ..
- * row0 + RW of this wave: rows are processed TT tokens at a time, and the
- * weight group loaded for them is reused by all TT. */
-template <int RW, int TT>
-__device__ __forceinline__ void gateup_rows(uint16_t *__restrict__ act,
-                                            const uint16_t *__restrict__ x,
-                                            const uint32_t *__restrict__ token_index,
-                                            const k3_moe_expert &ex, uint32_t base, uint32_t n,
-                                            uint32_t row0, uint32_t H, uint32_t F, uint32_t kind,
-                                            float beta, float lb) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t G = H / 32u;
-    const uint8_t *gp = (const uint8_t *)ex.gate_packed + (uint64_t)row0 * (H / 2u);
-    const uint8_t *up = (const uint8_t *)ex.up_packed + (uint64_t)row0 * (H / 2u);
-    const bool a16 = (((uintptr_t)gp | (uintptr_t)up) % 16u) == 0u;
-    const uint8_t *gsc = (const uint8_t *)ex.gate_scales + (uint64_t)row0 * G;
-    const uint8_t *usc = (const uint8_t *)ex.up_scales + (uint64_t)row0 * G;
-    for (uint32_t p0 = 0; p0 < n; p0 += TT) {
-        const uint32_t active = n - p0 < (uint32_t)TT ? n - p0 : (uint32_t)TT;
-        uint32_t tok[TT];
-#pragma unroll
-        for (int t = 0; t < TT; t++)
-            tok[t] = token_index[base + p0 + ((uint32_t)t < active ? (uint32_t)t : 0u)];
-        float acc[TT][2 * RW];
-#pragma unroll
-        for (int t = 0; t < TT; t++)
-#pragma unroll
-            for (int i = 0; i < 2 * RW; i++) acc[t][i] = 0.0f;
-        for (uint32_t g = lane; g < G; g += 64u) {
-            uint4 w[2 * RW];
-            float sc[2 * RW];
-#pragma unroll
-            for (int i = 0; i < RW; i++) {
-                w[i] = gload16(gp + (uint64_t)i * (H / 2u) + 16u * g, a16);
-                w[RW + i] = gload16(up + (uint64_t)i * (H / 2u) + 16u * g, a16);
-                sc[i] = e8m0_to_f32(gsc[(uint64_t)i * G + g]);
-                sc[RW + i] = e8m0_to_f32(usc[(uint64_t)i * G + g]);
-            }
-#pragma unroll
-            for (int t = 0; t < TT; t++) {
-                if ((uint32_t)t < active) {
-                    float xf[32];
-                    bf16x32_to_f32((const uint4 *)(x + (uint64_t)tok[t] * H) + 4u * g, xf);
-#pragma unroll
-                    for (int i = 0; i < 2 * RW; i++)
-                        acc[t][i] = fmaf(fp4_group(w[i], xf), sc[i], acc[t][i]);
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const float v = wave_sum_rows<2 * RW>(acc[t]);
-            const float uu = __shfl_xor(v, 32, 64);
-            const int owner = wave_rows_owner<2 * RW>();
-            if ((uint32_t)t < active && lane < 32u && (lane & (64u / (2u * RW) - 1u)) == 0u)
-                act[(uint64_t)(base + p0 + t) * F + row0 + owner] =
-                    f32_to_bf16(gated_act(bf16_round(v), bf16_round(uu), kind, beta, lb));
-        }
-    }
-}
-
-/* grid (up to F / (4 * RW), walk), block 256 (ExactWork); column blocks
- * past the grid's x extent are walked (the hand-off list, usually empty,
- * runs on a small grid). */
-template <int RW, int TT>
-__global__ __launch_bounds__(256, 2) void grouped_gateup_kernel(
-        uint16_t *__restrict__ act, const uint16_t *__restrict__ x, ExactWork W,
-        const uint32_t *__restrict__ token_index, const k3_moe_expert *__restrict__ experts,
-        uint32_t H, uint32_t F, uint32_t kind, float beta, float lb) {
-    const uint32_t nbx = F / (4u * RW);
-    const uint32_t listed = W.list ? *W.list_count : 0u;
-    if (W.list && blockIdx.y >= listed) return;
-    for (uint32_t bx = blockIdx.x; bx < nbx; bx += gridDim.x) {
-        const uint32_t row0 = (bx * 4u + (threadIdx.x >> 6)) * RW;
-        if (!W.list) {
-            uint32_t e, base, n;
-            for (uint32_t q = blockIdx.y; exact_tile(W, q, e, base, n); q += gridDim.y)
-                gateup_rows<RW, TT>(act, x, token_index, experts[e], base, n, row0, H, F, kind,
-                                    beta, lb);
-            continue;
-        }
-        for (uint32_t q = blockIdx.y; q < listed; q += gridDim.y) {
-            const uint32_t e = W.list[q];
-            gateup_rows<RW, TT>(act, x, token_index, experts[e], W.offsets[e], W.counts[e], row0,
-                                H, F, kind, beta, lb);
-        }
-    }
-}
-
-/* Down of plan rows [base, base + n) of expert e into their route slots of
- * y, weight rows row0 .. row0 + RB of this wave, TT tokens at a time. */
-template <int RB, int TT>
-__device__ __forceinline__ void down_rows(uint16_t *__restrict__ y,
-                                          const uint16_t *__restrict__ act,
-                                          const uint32_t *__restrict__ route_index,
-                                          const k3_moe_expert &ex, uint32_t base, uint32_t n,
-                                          uint32_t row0, uint32_t H, uint32_t F) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t G = F / 32u;
-    const uint8_t *dp = (const uint8_t *)ex.down_packed + (uint64_t)row0 * (F / 2u);
-    const bool a16 = ((uintptr_t)dp % 16u) == 0u;
-    const uint8_t *ds = (const uint8_t *)ex.down_scales + (uint64_t)row0 * G;
-    for (uint32_t p0 = 0; p0 < n; p0 += TT) {
-        const uint32_t active = n - p0 < (uint32_t)TT ? n - p0 : (uint32_t)TT;
-        float acc[TT][RB];
-#pragma unroll
-        for (int t = 0; t < TT; t++)
-#pragma unroll
-            for (int i = 0; i < RB; i++) acc[t][i] = 0.0f;
-        for (uint32_t g = lane; g < G; g += 64u) {
-            uint4 w[RB];
-            float sc[RB];
-#pragma unroll
-            for (int i = 0; i < RB; i++) {
-                w[i] = gload16(dp + (uint64_t)i * (F / 2u) + 16u * g, a16);
-                sc[i] = e8m0_to_f32(ds[(uint64_t)i * G + g]);
-            }
-#pragma unroll
-            for (int t = 0; t < TT; t++) {
-                if ((uint32_t)t < active) {
-                    float xf[32];
-                    bf16x32_to_f32((const uint4 *)(act + (uint64_t)(base + p0 + t) * F) + 4u * g, xf);
-#pragma unroll
-                    for (int i = 0; i < RB; i++)
-                        acc[t][i] = fmaf(fp4_group(w[i], xf), sc[i], acc[t][i]);
-                }
-            }
-        }
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const float v = wave_sum_rows<RB>(acc[t]);
-            const int owner = wave_rows_owner<RB>();
-            if ((uint32_t)t < active && (lane & (64u / RB - 1u)) == 0u)
-                y[(uint64_t)route_index[base + p0 + t] * H + row0 + owner] = f32_to_bf16(v);
-        }
-    }
-}
-
-/* grid (up to H / (4 * RB), walk), block 256: y[route] = down_e . act[row]
- * (column blocks walked as in grouped_gateup_kernel). Two
- * waves per SIMD (at most 256 VGPRs): at one wave per SIMD (269 VGPRs) the
- * kernel took 15.0 against 8.7 ms at cfg3. */
-template <int RB, int TT>
-__global__ __launch_bounds__(256, 2) void grouped_down_kernel(
-        uint16_t *__restrict__ y, const uint16_t *__restrict__ act, ExactWork W,
-        const uint32_t *__restrict__ route_index, const k3_moe_expert *__restrict__ experts,
-        uint32_t H, uint32_t F) {
-    const uint32_t nbx = H / (4u * RB);
-    const uint32_t listed = W.list ? *W.list_count : 0u;
-    if (W.list && blockIdx.y >= listed) return;
-    for (uint32_t bx = blockIdx.x; bx < nbx; bx += gridDim.x) {
-        const uint32_t row0 = (bx * 4u + (threadIdx.x >> 6)) * RB;
-        if (!W.list) {
-            uint32_t e, base, n;
-            for (uint32_t q = blockIdx.y; exact_tile(W, q, e, base, n); q += gridDim.y)
-                down_rows<RB, TT>(y, act, route_index, experts[e], base, n, row0, H, F);
-            continue;
-        }
-        for (uint32_t q = blockIdx.y; q < listed; q += gridDim.y) {
-            const uint32_t e = W.list[q];
-            down_rows<RB, TT>(y, act, route_index, experts[e], W.offsets[e], W.counts[e], row0,
-                              H, F);
-        }
-    }
-}
 
 /* out[t, d] = bf16(residual + bf16(sum_r w[t, r] * y[t*k + r, d])), rank
  * order, invalid routes skipped (k3_rocm_ops.cu:1452-1510). grid
@@ -604,19 +418,11 @@ DecodeParams decode_params(const Workspace &ws, void *output, const void *hidden
     return P;
 }
 
-/* Experts the MFMA path hands to the exact kernels (tensors not 8-byte
- * aligned) are walked by a grid of this many expert rows: with none, the
- * blocks exit at once. */
-constexpr uint32_t kFallbackExperts = 8;
-/* column blocks of the hand-off grid (each walks the rest): an empty list
- * then costs a launch of 8 x 32 blocks, not thousands */
-constexpr uint32_t kFallbackCols = 32;
-
 /* Expert stage on routes already in ws.ids / ws.weights. */
 bool run_experts(const Workspace &ws, void *output, const void *hidden, const void *residual,
                  const k3_moe_expert *experts, const k3_moe_shape &s, uint32_t T,
                  uint32_t precision, hipStream_t st, const StageMarker &mark) {
-    const uint32_t H = s.hidden, F = s.ffn, E = s.expert_count, k = s.top_k;
+    const uint32_t H = s.hidden, E = s.expert_count, k = s.top_k;
     const float beta = s.activation == 1u ? 1.0f : s.beta;
     const float lb = s.activation == 1u ? 1.0f : s.linear_beta;
     if (T == 1u && decode_supported(s)) { /* every precision: exact decode */
@@ -628,12 +434,8 @@ bool run_experts(const Workspace &ws, void *output, const void *hidden, const vo
     if (!launch_plan(ws.counts, ws.offsets, ws.unique, ws.summary, ws.token_index,
                      ws.route_index, ws.chunk_base, ws.ids, T, k, E, st))
         return false;
-    const uint32_t upper = (uint64_t)T * k < E ? T * k : E;
-    /* weight rows per wave and tokens per weight load: gate/up 2 x 2
-     * (255 VGPRs), down 4 x 4 (two waves per SIMD). Measured against 4 x 4
-     * / 2 x 2 / 2 x 1 / 1 x 2 shapes on cfg3 and cfg4: 26.5 and 387 ms per
-     * layer, the next best 29.2 and 419 ms. */
-    constexpr int RW = 2, TT = 2, RB = 4, TD = 4;
+    ExactGroup g = ws.exact;
+    g.experts = experts;
     if (precision != K3_MOE_EXACT) {
         if (!mfma_launch_experts(ws.mfma, ws.y, (const uint16_t *)hidden, ws.counts, ws.offsets,
                                  ws.token_index, ws.route_index, experts, s, T,
@@ -642,20 +444,10 @@ bool run_experts(const Workspace &ws, void *output, const void *hidden, const vo
         /* experts with a tensor that is not 8-byte aligned (no MFMA tiles):
          * the exact kernels, after the MFMA down kernel has consumed the
          * activation codes that share `act` */
-        const uint32_t walk = upper < kFallbackExperts ? upper : kFallbackExperts;
-        const uint32_t gx = F / (4u * RW) < kFallbackCols ? F / (4u * RW) : kFallbackCols;
-        const uint32_t dx = H / (4u * RB) < kFallbackCols ? H / (4u * RB) : kFallbackCols;
-        ExactWork W{};
-        W.list_count = ws.mfma.unaligned;
-        W.list = ws.mfma.unaligned + 1;
-        W.counts = ws.counts;
-        W.offsets = ws.offsets;
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(grouped_gateup_kernel<RW, TT>),
-                           dim3(gx, walk), dim3(256), 0, st, ws.act,
-                           (const uint16_t *)hidden, W, ws.token_index, experts, H, F,
-                           s.activation, beta, lb);
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(grouped_down_kernel<RB, TD>), dim3(dx, walk),
-                           dim3(256), 0, st, ws.y, ws.act, W, ws.route_index, experts, H, F);
+        g.list = ws.mfma.unaligned;
+        if (!launch_exact_gateup(g, ws.act, (const uint16_t *)hidden, s.activation, beta, lb, st) ||
+            !launch_exact_down(g, ws.y, ws.act, st))
+            return false;
         mark(K3_MOE_STAGE_COMBINE);
         hipLaunchKernelGGL(combine_kernel, dim3((H / 8u + kCombineThreads - 1u) / kCombineThreads, T),
                            dim3(kCombineThreads), 0, st, (uint16_t *)output, ws.y,
@@ -664,20 +456,11 @@ bool run_experts(const Workspace &ws, void *output, const void *hidden, const vo
         return hipGetLastError() == hipSuccess;
     }
     mark(K3_MOE_STAGE_GATE_UP);
-    /* exact: workgroups over the tile lists of every selected expert */
-    if (!build_tiles_all(ws.mfma, ws.counts, ws.offsets, experts, E, st)) return false;
-    ExactWork W{};
-    W.tiles = ws.mfma.tiles;
-    W.tile_count = ws.mfma.tile_count;
-    for (int c = 0; c < kTileClasses; c++) W.cap[c] = ws.mfma.tile_cap[c];
-    W.counts = ws.counts;
-    W.offsets = ws.offsets;
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(grouped_gateup_kernel<RW, TT>), dim3(F / (4u * RW), upper),
-                       dim3(256), 0, st, ws.act, (const uint16_t *)hidden, W, ws.token_index,
-                       experts, H, F, s.activation, beta, lb);
+    if (!launch_exact_tiles(g, st) ||
+        !launch_exact_gateup(g, ws.act, (const uint16_t *)hidden, s.activation, beta, lb, st))
+        return false;
     mark(K3_MOE_STAGE_DOWN);
-    hipLaunchKernelGGL(HIP_KERNEL_NAME(grouped_down_kernel<RB, TD>), dim3(H / (4u * RB), upper),
-                       dim3(256), 0, st, ws.y, ws.act, W, ws.route_index, experts, H, F);
+    if (!launch_exact_down(g, ws.y, ws.act, st)) return false;
     mark(K3_MOE_STAGE_COMBINE);
     hipLaunchKernelGGL(combine_kernel, dim3((H / 8u + kCombineThreads - 1u) / kCombineThreads, T),
                        dim3(kCombineThreads), 0, st, (uint16_t *)output, ws.y,
