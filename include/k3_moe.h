@@ -32,10 +32,9 @@ extern "C" {
  * [rows, columns / 32]. Fields follow the six-tensor span order of
  * k3_prefill.c:71-75 (w1 = gate, w2 = down, w3 = up). Tensors must start
  * 8-byte aligned; the 8-mod-16 starts of real checkpoint spans
- * (k3_rocm_ops.cu:207-223) are read as 8-byte pairs by the exact kernels
- * and as 16-byte direct-to-LDS pieces (which take 8-byte aligned sources
- * on gfx950) by the MFMA kernels, with the same results as aligned
- * tensors.
+ * (k3_rocm_ops.cu:207-223) are read as 8-byte pairs by the decode kernels
+ * and as 16-byte direct-to-LDS pieces (which take unaligned sources on
+ * gfx950) by the batch kernels, with the same results as aligned tensors.
  */
 typedef struct {
     const void *gate_packed;  /* w1.weight_packed [ffn, hidden / 2]  */
@@ -55,8 +54,9 @@ typedef enum {
 } k3_moe_activation;
 
 typedef enum {
-    /* Fixed wave64 fp32 orders on the vector ALUs: bit-identical to the
-     * CPU oracle, to the per-matrix k3_rocm_mxfp4_* entry points and
+    /* Fixed wave64 fp32 orders (one token on the vector units, batches on
+     * the fp32 matrix units, whose K = 1 products are the same rounded
+     * fmaf chain): bit-identical to the CPU oracle, to the per-matrix k3_rocm_mxfp4_* entry points and
      * between decode and any batch size. */
     K3_MOE_EXACT = 0,
     /* Grouped GEMM on CDNA4 scaled MFMA for token_count > 1: weights stay
@@ -132,7 +132,7 @@ bool k3_moe_router_choices_f32(float *choices, const float *logits, const float 
  * Routes of a token batch, replacing the prefill router pair
  * k3_rocm_bf16_gemm_f32 + k3_rocm_router_topk_f32_batch
  * (k3_engine_prefill.inc:1448-1460) with the same ids and weights, bit for
- * bit. From 32 tokens on (hidden % 64 == 0, hidden <= 8192, expert_count
+ * bit. From 80 tokens on (hidden % 64 == 0, hidden <= 8192, expert_count
  * <= 1024, 16-byte aligned hidden and router_weight) the logits run on bf16
  * MFMA and each token recomputes in the exact order only the experts that a
  * rigorous error bound cannot rule out of its top-k; otherwise the exact

@@ -219,6 +219,85 @@ bool launch_bf16_rows_ref(float *out, const void *w, const void *x, uint32_t tok
 }
 
 /*
+ * The same logits for several tokens from 16-byte rows: a wave has two weight
+ * rows and TT tokens, so a row's chunk is read once for TT tokens and a
+ * token's once for two rows (one row per wave read every token's row for each
+ * of its rows: at 5 tokens 896 x 5 x 14 KB through the L1s for 12.8 MB of
+ * weights). Chunks with j even belong to the partials 2 lane and 2 lane + 1,
+ * odd ones to those + 128, so two waves take one parity each; the odd one's
+ * partials cross in LDS for the tree's level 128 and the even one finishes as
+ * bf16_rows_ref_kernel. Bound by the quads' five vector instructions from
+ * about 64 tokens on. K3 router (896 x 7168), before -> after: 2 tokens 14.5 ->
+ * 8.0 us, 5 tokens 28 -> 9.9, 20 tokens 75 -> 12.8, 64 tokens 178 -> 24; and
+ * against a register-blocked GEMM of 16 x 8 tiles in the same order, 512
+ * tokens 237 -> 156, 8192 tokens 3750 -> 2359.
+ */
+template <int TT>
+__global__ __launch_bounds__(256) void bf16_rows_ref_pair_kernel(
+        float *__restrict__ out, const uint16_t *__restrict__ weights,
+        const uint16_t *__restrict__ input, uint32_t tokens, uint32_t rows, uint32_t cols) {
+    constexpr int R = 2, N = 2 * R * TT; /* partials of a wave: (row, token, quad) */
+    __shared__ float odd[2][N][64];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t parity = wave & 1u, pair = wave >> 1;
+    const uint32_t row0 = (blockIdx.x * 2u + pair) * R, t0 = blockIdx.y * TT;
+    const uint32_t chunks = cols / 8u;
+    const uint4 *w4[R], *x4[TT]; /* past the end: the last row / token again */
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const uint32_t row = row0 + (uint32_t)r < rows ? row0 + (uint32_t)r : rows - 1u;
+        w4[r] = (const uint4 *)(weights + (uint64_t)row * cols);
+    }
+#pragma unroll
+    for (int t = 0; t < TT; t++) {
+        const uint32_t tok = t0 + (uint32_t)t < tokens ? t0 + (uint32_t)t : tokens - 1u;
+        x4[t] = (const uint4 *)(input + (uint64_t)tok * cols);
+    }
+    float p[N];
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = 0.0f;
+    for (uint32_t c = lane + 64u * parity; c < chunks; c += 128u) {
+        uint4 wv[R], xv[TT];
+#pragma unroll
+        for (int r = 0; r < R; r++) wv[r] = w4[r][c];
+#pragma unroll
+        for (int t = 0; t < TT; t++) xv[t] = x4[t][c];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int t = 0; t < TT; t++) {
+                float *q = p + 2 * (r * TT + t);
+                q[0] = __fadd_rn(q[0], ref_quad(wv[r].x, wv[r].y, xv[t].x, xv[t].y));
+                q[1] = __fadd_rn(q[1], ref_quad(wv[r].z, wv[r].w, xv[t].z, xv[t].w));
+            }
+    }
+    if (parity) {
+#pragma unroll
+        for (int i = 0; i < N; i++) odd[pair][i][lane] = p[i];
+    }
+    __syncthreads();
+    if (parity) return;
+#pragma unroll
+    for (int i = 0; i < N; i++) p[i] = __fadd_rn(p[i], odd[pair][i][lane]); /* level 128 */
+    float v = wave_sum_rows<N>(p); /* levels 64 .. 2 */
+    constexpr int kPer = 64 / N;   /* lanes per partial */
+    v = __fadd_rn(v, __shfl_xor(v, kPer, 64));
+    const uint32_t owner = (uint32_t)wave_rows_owner<N>() / 2u;
+    const uint32_t row = row0 + owner / TT, tok = t0 + owner % TT;
+    if ((lane & (2u * kPer - 1u)) == 0u && row < rows && tok < tokens)
+        out[(uint64_t)tok * rows + row] = v;
+}
+
+template <int TT>
+bool launch_bf16_rows_ref_pair(float *out, const void *w, const void *x, uint32_t tokens,
+                               uint32_t rows, uint32_t cols, hipStream_t s) {
+    dim3 grid((rows + 3u) / 4u, (tokens + TT - 1u) / TT);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(bf16_rows_ref_pair_kernel<TT>), grid, dim3(kThreads), 0, s,
+                       out, (const uint16_t *)w, (const uint16_t *)x, tokens, rows, cols);
+    return hipGetLastError() == hipSuccess;
+}
+
+/*
  * The same w64 order for many tokens at once (router logits of a prefill
  * batch), as a register-blocked GEMM: a block computes 32 tokens x 16 rows.
  * Wave w (of 8) owns tokens 8 (w / 2) .. +8 and rows 8 (w % 2) .. +8; lane l
@@ -358,147 +437,6 @@ bool launch_bf16_gemm_w64(void *out, const void *w, const void *x, uint32_t toke
                                 : (uint64_t)token_tiles * row_tiles;
     if (blocks > 0x7fffffffull) return false;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(bf16_gemm_w64_kernel<B16>), dim3((uint32_t)blocks), dim3(kGThreads), 0, s, out,
-                       (const uint16_t *)w, (const uint16_t *)x, tokens, rows, cols, row_tiles,
-                       xcd);
-    return hipGetLastError() == hipSuccess;
-}
-
-/*
- * Router logits of many tokens (f32, T >= 128) in the reference's order as
- * a blocked GEMM: a block computes 16 tokens x 8 weight rows; a K step is
- * 1024 columns (256 quads), so each of the reference's 256 partials of an
- * output gets exactly one quad per step. Wave w takes partials 64 (w % 4) +
- * lane (its K quarter) of tokens 8 (w / 4) .. + 8 and all 8 rows: one
- * accumulator per output, the quad summed by ref_quad, the quads of a
- * partial in K order as the reference's thread adds them. At the end the
- * K quarters meet in LDS as the reference's tree levels 128 (quarters q
- * and q + 2) and 64 (quarters 0 and 1), and wave_sum_rows<64> does levels
- * 32 .. 1. Out-of-range tokens/rows/columns stage zeros: a zero quad adds
- * +0, which changes no partial (a partial is never -0). The step's bf16
- * tiles are loaded into registers one step ahead and staged in LDS as fp32
- * quads, so each fragment read is one lane-contiguous ds_read_b128. Block
- * order is XCD-aware as in bf16_gemm_w64_kernel.
- */
-constexpr int kQT = 16, kQE = 8, kQThreads = 512;
-
-__device__ __forceinline__ float ref_quad_f4(const float4 &w, const float4 &x) {
-    const float p2 = __fmul_rn(w.z, x.z), p3 = __fmul_rn(w.w, x.w);
-    return __fadd_rn(fmaf(w.y, x.y, p2), fmaf(w.x, x.x, p3));
-}
-
-__global__ __launch_bounds__(512) void bf16_gemm_ref_kernel(
-        float *__restrict__ out, const uint16_t *__restrict__ weights,
-        const uint16_t *__restrict__ input, uint32_t tokens, uint32_t rows, uint32_t cols,
-        uint32_t row_tiles, uint32_t xcd_groups) {
-    __shared__ float4 xs[kQT][256];
-    __shared__ float4 wsm[kQE][256];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    uint32_t tt, et;
-    {
-        const uint32_t L = blockIdx.x;
-        if (xcd_groups) {
-            const uint32_t x = L & 7u, j = L >> 3;
-            const uint32_t base = row_tiles >> 3, rem = row_tiles & 7u;
-            const uint32_t cnt = base + (x < rem ? 1u : 0u);
-            const uint32_t start = x * base + (x < rem ? x : rem);
-            const uint32_t token_tiles = (tokens + kQT - 1u) / kQT;
-            if (cnt == 0u || j >= token_tiles * cnt) return;
-            tt = j / cnt;
-            et = start + j % cnt;
-        } else {
-            tt = L / row_tiles;
-            et = L % row_tiles;
-        }
-    }
-    const uint32_t t0 = tt * kQT, e0 = et * kQE;
-    const uint32_t chunks = cols / 8u, nsteps = (chunks + 127u) / 128u;
-    const uint4 *x4 = (const uint4 *)input, *w4 = (const uint4 *)weights;
-    /* staging items: 16 token rows then 8 weight rows, 128 chunks each */
-    constexpr int kItems = (kQT + kQE) * 128 / kQThreads;
-    uint4 reg[kItems];
-    auto load_step = [&](uint32_t s) {
-#pragma unroll
-        for (int q = 0; q < kItems; q++) {
-            const uint32_t it = tid + (uint32_t)q * kQThreads;
-            const uint32_t r = it >> 7, c = 128u * s + (it & 127u);
-            uint4 v = make_uint4(0u, 0u, 0u, 0u);
-            if (r < (uint32_t)kQT) {
-                if (t0 + r < tokens && c < chunks) v = x4[(uint64_t)(t0 + r) * chunks + c];
-            } else if (e0 + r - kQT < rows && c < chunks) {
-                v = w4[(uint64_t)(e0 + r - kQT) * chunks + c];
-            }
-            reg[q] = v;
-        }
-    };
-    const uint32_t kq = wave & 3u, tg = wave >> 2, qi = 64u * kq + lane;
-    float acc[64];
-#pragma unroll
-    for (int i = 0; i < 64; i++) acc[i] = 0.0f;
-    load_step(0u);
-    for (uint32_t s = 0; s < nsteps; s++) {
-        __syncthreads(); /* the previous step's reads are done */
-#pragma unroll
-        for (int q = 0; q < kItems; q++) {
-            const uint32_t it = tid + (uint32_t)q * kQThreads;
-            const uint4 v = reg[q];
-            const float4 a = make_float4(bf16_lo(v.x), bf16_hi(v.x), bf16_lo(v.y), bf16_hi(v.y));
-            const float4 b = make_float4(bf16_lo(v.z), bf16_hi(v.z), bf16_lo(v.w), bf16_hi(v.w));
-            const uint32_t r = it >> 7, c = it & 127u;
-            float4 *dst = r < (uint32_t)kQT ? &xs[r][2u * c] : &wsm[r - kQT][2u * c];
-            dst[0] = a;
-            dst[1] = b;
-        }
-        __syncthreads();
-        if (s + 1u < nsteps) load_step(s + 1u);
-        float4 wv[kQE];
-#pragma unroll
-        for (int e = 0; e < kQE; e++) wv[e] = wsm[e][qi];
-#pragma unroll
-        for (int t = 0; t < 8; t++) {
-            const float4 xv = xs[8u * tg + t][qi];
-#pragma unroll
-            for (int e = 0; e < kQE; e++)
-                acc[8 * t + e] = __fadd_rn(acc[8 * t + e], ref_quad_f4(wv[e], xv));
-        }
-    }
-    /* tree levels 128 and 64 across the K quarters, through LDS */
-    float *red = (float *)&xs[0][0]; /* [2 token groups][2][64 outputs][64 lanes] */
-    __syncthreads();
-    if (kq >= 2u) {
-#pragma unroll
-        for (int i = 0; i < 64; i++) red[((tg * 2u + kq - 2u) * 64u + i) * 64u + lane] = acc[i];
-    }
-    __syncthreads();
-    if (kq < 2u) {
-#pragma unroll
-        for (int i = 0; i < 64; i++)
-            acc[i] = __fadd_rn(acc[i], red[((tg * 2u + kq) * 64u + i) * 64u + lane]);
-    }
-    __syncthreads();
-    if (kq == 1u) {
-#pragma unroll
-        for (int i = 0; i < 64; i++) red[(tg * 64u + i) * 64u + lane] = acc[i];
-    }
-    __syncthreads();
-    if (kq != 0u) return;
-#pragma unroll
-    for (int i = 0; i < 64; i++) acc[i] = __fadd_rn(acc[i], red[(tg * 64u + i) * 64u + lane]);
-    const float v = wave_sum_rows<64>(acc);
-    const int owner = wave_rows_owner<64>();
-    const uint32_t t = t0 + 8u * tg + (uint32_t)(owner >> 3);
-    const uint32_t e = e0 + (uint32_t)(owner & 7);
-    if (t < tokens && e < rows) out[(uint64_t)t * rows + e] = v;
-}
-
-bool launch_bf16_gemm_ref(float *out, const void *w, const void *x, uint32_t tokens,
-                          uint32_t rows, uint32_t cols, hipStream_t s) {
-    const uint32_t token_tiles = (tokens + kQT - 1u) / kQT;
-    const uint32_t row_tiles = (rows + kQE - 1u) / kQE;
-    const uint32_t xcd = row_tiles >= 8u ? 1u : 0u;
-    const uint64_t blocks = xcd ? 8ull * token_tiles * ((row_tiles + 7u) / 8u)
-                                : (uint64_t)token_tiles * row_tiles;
-    if (blocks > 0x7fffffffull) return false;
-    hipLaunchKernelGGL(bf16_gemm_ref_kernel, dim3((uint32_t)blocks), dim3(kQThreads), 0, s, out,
                        (const uint16_t *)w, (const uint16_t *)x, tokens, rows, cols, row_tiles,
                        xcd);
     return hipGetLastError() == hipSuccess;
@@ -1063,10 +1001,11 @@ namespace {
 /* f32 router logits: the reference's order on every path */
 bool launch_bf16_ref_any(float *out, const void *w, const void *x, uint32_t tokens,
                          uint32_t rows, uint32_t cols, hipStream_t s) {
+    const bool vec = cols % 8u == 0u && ((uintptr_t)w | (uintptr_t)x) % 16u == 0u;
     if (tokens == 1u) return launch_bf16_rows_ref<1>(out, w, x, 1u, rows, cols, s);
+    if (vec && tokens <= 4u) return launch_bf16_rows_ref_pair<4>(out, w, x, tokens, rows, cols, s);
+    if (vec) return launch_bf16_rows_ref_pair<8>(out, w, x, tokens, rows, cols, s);
     if (tokens <= 4u) return launch_bf16_rows_ref<4>(out, w, x, tokens, rows, cols, s);
-    if (tokens >= kGemmMinTokens && cols % 8u == 0u && ((uintptr_t)w | (uintptr_t)x) % 16u == 0u)
-        return launch_bf16_gemm_ref(out, w, x, tokens, rows, cols, s);
     return launch_bf16_rows_ref<16>(out, w, x, tokens, rows, cols, s);
 }
 
