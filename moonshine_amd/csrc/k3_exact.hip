@@ -70,9 +70,15 @@ struct BlockRows {
     }
 };
 
+/* 16 bytes a lane into consecutive LDS from a wave-uniform LDS address (a
+ * number: from a pointer the compiler tests it for null at every use). */
+__device__ __forceinline__ void dma16(const uint8_t *src, uint32_t lds) {
+    __builtin_amdgcn_global_load_lds((const void *)src, (lds_void *)(uintptr_t)lds, 16, 0, 0);
+}
+
 /* What a block carries from one tile to the next. */
 struct Pipe {
-    uint8_t *lds;  /* ring, then two scale buffers */
+    uint32_t lds;  /* LDS address of the ring, then two scale buffers */
     uint32_t slot; /* ring slot of the tile's stage 0 */
     uint32_t buf;  /* its scale buffer */
     bool primed;   /* stages 0 and 1 and the scales are on their way */
@@ -166,7 +172,9 @@ struct Core {
         }
     }
     static __device__ __forceinline__ float scale(uint32_t raw) {
-        if constexpr (std::is_same<Fmt, Mx4>::value) return e8m0_to_f32(raw);
+        /* e8m0_to_f32 in one instruction: 2^-127 2^raw, +inf at 255 */
+        if constexpr (std::is_same<Fmt, Mx4>::value)
+            return __builtin_amdgcn_ldexpf(__uint_as_float(0x00400000u), (int)raw);
         else return __uint_as_float(raw);
     }
 
@@ -177,14 +185,14 @@ struct Core {
     }
 
     /* Whole rows' scales, contiguous bytes per half. */
-    static __device__ __forceinline__ void fetch_scales(uint8_t *sc, const BlockRows &R,
+    static __device__ __forceinline__ void fetch_scales(uint32_t sc, const BlockRows &R,
                                                         uint32_t G, uint32_t w, uint32_t L) {
         constexpr uint32_t kHalf = RB < 32 ? RB : 32; /* rows from s[0] */
         const uint32_t half = kHalf * G / 16u, all = RB * G / 16u;
         for (uint32_t i = 64u * w; i < all; i += 64u * W) {
             uint32_t p = i + L;
             p = p < all ? p : all - 1u;
-            dma<16>(p < half ? R.s[0] + 16u * p : R.s[1] + 16u * (p - half), sc + 16u * i);
+            dma16(p < half ? R.s[0] + 16u * p : R.s[1] + 16u * (p - half), sc + 16u * i);
         }
     }
 
@@ -203,22 +211,26 @@ struct Core {
         constexpr uint32_t kRowPieces = SB / 16;
         const uint32_t dr = kDmaRows * w + L / kRowPieces;
         const uint32_t dp = (L % kRowPieces) ^ (dr & 15u);
-        uint32_t voff[kDma];
+        /* the lane's offset from its half's first row; in a partial last stage
+         * the pieces past the row's end repeat its last one */
+        uint32_t voff[kDma], vend[kDma];
+        const uint32_t pieces = rbytes / 16u, rest = pieces % kRowPieces;
+        const uint32_t whole = pieces / kRowPieces;
 #pragma unroll
-        for (int m = 0; m < kDma; m++)
+        for (int m = 0; m < kDma; m++) {
             voff[m] = R.row(dr + kDmaRows * W * (uint32_t)m) * rbytes + 16u * dp;
-        uint8_t *const ring = pipe.lds;
+            vend[m] = dp < rest ? voff[m] : voff[m] - 16u * (dp + 1u - rest);
+        }
+        const uint32_t ring = __builtin_amdgcn_readfirstlane(pipe.lds);
         /* no branches: the waits on the token columns count these loads */
         auto fetch = [&](const uint8_t *w0, const uint8_t *w1, uint32_t s, uint32_t slot) {
-            const int left = (int)(rbytes / 16u - kRowPieces * s); /* pieces from s on */
-            /* past the row's end its last piece is repeated */
-            const int over = (int)dp - left + 1;
-            const uint32_t back = 16u * (uint32_t)(over > 0 ? over : 0);
-            uint8_t *const dst = ring + kStage * slot + 1024u * w;
+            const uint32_t dst = ring + kStage * slot + 1024u * w;
+            const bool last = s == whole;
 #pragma unroll
             for (int m = 0; m < kDma; m++)
-                dma<16>((m * kDmaRows * W >= 32u ? w1 : w0) + (uint64_t)s * SB + (voff[m] - back),
-                        dst + 1024u * W * m);
+                dma16((m * kDmaRows * W >= 32u ? w1 : w0) + (uint64_t)s * SB +
+                          (last ? vend[m] : voff[m]),
+                      dst + 1024u * W * m);
         };
         /* A: lane 4 c + i (of RB lanes) holds kC columns of token i: of the
          * wave's group c / kLG, columns kC (c % kLG) .. */
@@ -242,12 +254,12 @@ struct Core {
         for (int q = 0; q < kGW; q++)
 #pragma unroll
             for (int i = 0; i < kPieces; i++)
-                at[q][i] = lds_addr(ring) + SB * (L % RB) +
+                at[q][i] = ring + SB * (L % RB) +
                            (((kPieces * (w + W * (uint32_t)q) + (uint32_t)i) ^ (L & 15u)) << 4);
         for (uint32_t g0 = 0; g0 < G; g0 += kScaleGroups) {
             const uint32_t gn = G - g0 < kScaleGroups ? G - g0 : kScaleGroups;
             const uint32_t s_end = (g0 + gn + kSG - 1u) / kSG, s_begin = g0 / kSG;
-            uint8_t *const sc = ring + kRing * kStage + kScaleBytes * pipe.buf;
+            const uint32_t sc = ring + kRing * kStage + kScaleBytes * pipe.buf;
             if (!pipe.primed) {
                 wait_vm<0>();
                 __syncthreads(); /* the last reads of what is filled now are done */
@@ -257,7 +269,9 @@ struct Core {
                     const uint32_t r = L % RB;
                     const uint8_t *row = (r < 32u ? R.s[0] : R.s[1]) + (uint64_t)R.row(r) * G + g0;
 #pragma unroll 1
-                    for (uint32_t i = w; i < gn; i += W) sc[gn * r + i] = row[i];
+                    for (uint32_t i = w; i < gn; i += W)
+                        *(__attribute__((address_space(3))) uint8_t *)(uintptr_t)(sc + gn * r + i) =
+                            row[i];
                     __syncthreads();
                 }
                 fetch(R.w[0], R.w[1], s_begin, pipe.slot);
@@ -265,11 +279,11 @@ struct Core {
                 fetch(R.w[0], R.w[1], s_begin + 1u < s_end ? s_begin + 1u : s_begin, s1);
             }
             pipe.primed = false;
-            const uint32_t sc_lds = lds_addr(sc) + gn * (L % RB) + w;
+            const uint32_t sc_lds = sc + gn * (L % RB) + w;
             Columns xs;
             load_x(xs, X, xat(s_begin));
             wait_vm<0>(); /* here, so that the loop's own waits need not drain */
-            uint32_t slot = pipe.slot;
+            uint32_t slot = __builtin_amdgcn_readfirstlane(pipe.slot);
             auto step = [&](uint32_t s, auto SM) { /* false after the last stage */
                 /* only the next stage's DMA stays in flight */
                 wait_vm<kDma>();
@@ -387,7 +401,7 @@ struct Core {
     static __device__ __forceinline__ uint32_t meet(const Pipe &pipe, const Result &v) {
         const uint32_t w = threadIdx.x >> 6, L = threadIdx.x & 63u;
         const uint32_t last = pipe.slot >= 1u ? pipe.slot - 1u : kRing - 1u;
-        const uint32_t red = lds_addr(pipe.lds) + kStage * last;
+        const uint32_t red = pipe.lds + kStage * last;
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier(); /* the stage's last reads are done */
         asm volatile("" ::: "memory");
@@ -630,7 +644,7 @@ __global__ __launch_bounds__(512, Heavy ? 2 : 4) void exact_tiles_run_kernel(Arg
     /* short rows (a stage or less) and many scales: no look-ahead */
     const bool ahead = G <= kScaleGroups && G > SB / 16;
     Walk p{blockIdx.x, 0u};
-    Pipe pipe{smem, 0u, 0u, false};
+    Pipe pipe{lds_addr(smem), 0u, 0u, false};
     Tile T, N;
     bool have = next_tile<Heavy>(A, p, T);
     while (have) {
@@ -726,7 +740,7 @@ __global__ __launch_bounds__(512, 2 * dense_blocks(RB, NT)) void exact_dense_ker
     constexpr uint32_t TT = C::kTokens;
     const uint32_t G = A.cols / 32u;
     const bool ahead = G <= kScaleGroups && G > (uint32_t)C::kSG;
-    Pipe pipe{smem, 0u, 0u, false};
+    Pipe pipe{lds_addr(smem), 0u, 0u, false};
     BlockRows R, N;
     uint32_t r0, t0, nr0, nt0, wk = blockIdx.x;
     bool have = dense_tile<Fmt, RB, TT>(A, wk, r0, t0, R);
