@@ -24,6 +24,7 @@
  */
 #include "k3_device.h"
 #include "k3_internal.h"
+#include "k3_lds.h"
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -58,7 +59,8 @@ __device__ __forceinline__ uint4 codes_to_bf16(uint2 v) {
         for (int p = 0; p < 2; p++) {
             const float lo = (float)(int8_t)(u[h] >> (16 * p));
             const float hi = (float)(int8_t)(u[h] >> (16 * p + 8));
-            o[2 * h + p] = (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xffff0000u);
+            /* the two upper halves */
+            o[2 * h + p] = __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
         }
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
@@ -223,6 +225,175 @@ __global__ __launch_bounds__(512) void proj_mfma_kernel(ProjArgs P) {
         }
 }
 
+/*
+ * The Q8-128 form for many tokens: block tile 256 tokens x 128 rows, eight
+ * waves of 64 x 64, so a stage of 64 columns (32 KB of tokens, 16 KB of codes
+ * as bf16) feeds 32 MFMAs a wave from 16 LDS reads (the 32 x 64 wave tile
+ * above reads 12 for 16, and its LDS reads outlast its MFMAs). Three stages:
+ * tokens by direct-to-LDS loads two stages ahead (whole 128-byte lines,
+ * swizzled as the expert kernels' A tiles), codes into registers two stages
+ * ahead, converted and written one ahead, after the stage's MFMAs. LDS
+ * accesses and their waits are explicit: the compiler would drain the loads
+ * in flight before each. 2048 tokens, before -> after, us: 6144 x 7168
+ * 308 -> 251, 7168 x 3584 201 -> 127; 8192 tokens 1231 -> 805, 724 -> 468.
+ */
+constexpr uint32_t kWT = 256, kWN = 128;              /* block tile */
+constexpr uint32_t kWA = kWT * 128u, kWB = kWN * 128u; /* bytes of a stage */
+
+/* Both kernels hold one block a CU, and a round of tiles over the 256 CUs
+ * takes the wide one 6/5 as long for twice the work (7168 columns: 123 and
+ * 103 us, 1024 columns: 21 and 17 us): wide where that pays for its rounds. */
+static bool wide_pays(uint32_t T, uint32_t N) {
+    auto rounds = [&](uint32_t tt) {
+        return ((T + tt - 1u) / tt * (uint64_t)((N + 127u) / 128u) + 255u) / 256u;
+    };
+    return 6u * rounds(kWT) < 5u * rounds(kPT);
+}
+
+__global__ __launch_bounds__(512, 2) void proj_wide_kernel(ProjArgs P) {
+    __shared__ __attribute__((aligned(16))) uint8_t smem[3u * (kWA + kWB)];
+    const uint32_t T = P.T, N = P.N, K = P.K;
+    const uint32_t ntt = (T + kWT - 1u) / kWT, nnt = (N + kWN - 1u) / kWN;
+    const uint32_t works = ntt * nnt, per = (works + 7u) / 8u;
+    const uint32_t j8 = blockIdx.x >> 3, wk = (blockIdx.x & 7u) * per + j8;
+    if (j8 >= per || wk >= works) return;
+    const uint32_t t0 = (wk / nnt) * kWT, n0 = (wk % nnt) * kWN;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t wm = wave >> 1, wn = wave & 1u, g = lane >> 4, c = lane & 15u;
+    const uint32_t lds = lds_addr(smem);
+    /* tokens: wave w fills rows 32 w .. + 32 (four 8-row chunks); rows past
+     * T repeat the last one (not stored) */
+    const uint8_t *xs[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) {
+        const uint32_t h = (uint32_t)m & 1u;
+        const uint32_t r = t0 + 32u * wave + 16u * ((uint32_t)m >> 1) + a_dma_row(lane, h);
+        xs[m] = (const uint8_t *)P.x + 2ull * (r < T ? r : T - 1u) * K + 16u * a_dma_piece(lane, h);
+    }
+    /* codes: thread t loads 16 of row t / 4 per stage */
+    const uint32_t br = tid >> 2, bq = tid & 3u;
+    const uint8_t *ws = (const uint8_t *)P.w + (uint64_t)(n0 + br < N ? n0 + br : N - 1u) * K + 16u * bq;
+    const uint32_t b_dst = kWA + 2048u * (br >> 4) + a_slot(br & 15u, 2u * bq);
+    const uint32_t b_dst2 = kWA + 2048u * (br >> 4) + a_slot(br & 15u, 2u * bq + 1u);
+    const uint32_t nblk = K / 128u, nsteps = K / kPK, last = nsteps - 1u;
+    const float *srow[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t r = n0 + 64u * wn + 16u * (uint32_t)j + c;
+        srow[j] = P.scales + (uint64_t)(r < N ? r : N - 1u) * nblk;
+    }
+    auto fetch = [&](uint32_t s, uint32_t slot) { /* past the end: the last stage again */
+        const uint32_t off = 128u * (s < last ? s : last);
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            __builtin_amdgcn_global_load_lds(
+                (const void *)(xs[m] + off),
+                (lds_void *)(uintptr_t)(lds + (kWA + kWB) * slot + 4096u * wave + 1024u * m), 16, 0,
+                0);
+    };
+    auto codes = [&](uint32_t s) { return *(const u32x4_t *)(ws + kPK * (s < last ? s : last)); };
+    auto write = [&](const u32x4_t &q, uint32_t slot) {
+        const uint32_t base = lds + (kWA + kWB) * slot;
+        const uint4 lo = codes_to_bf16(make_uint2(q[0], q[1])), hi = codes_to_bf16(make_uint2(q[2], q[3]));
+        const u32x4_t l = {lo.x, lo.y, lo.z, lo.w}, h = {hi.x, hi.y, hi.z, hi.w};
+        asm volatile("ds_write_b128 %0, %1\n\tds_write_b128 %2, %3" ::"v"(base + b_dst), "v"(l),
+                     "v"(base + b_dst2), "v"(h)
+                     : "memory");
+    };
+    f32x4_t acc[4][4], blk[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    /* the fragments of 32 columns: rows 64 wm + 16 i + c and 64 wn + 16 j + c */
+    const uint32_t a_base = lds + 2048u * 4u * wm, b_base = lds + kWA + 2048u * 4u * wn;
+    const uint32_t slot0 = a_slot(c, g), slot1 = a_slot(c, 4u + g);
+    float sc[4];
+    u32x4_t q0 = codes(0u), q1 = codes(1u);
+    write(q0, 0u);
+    asm volatile("" : "+v"(q1) : : "memory");
+    fetch(0u, 0u);
+    asm volatile("" ::: "memory");
+    q0 = codes(2u); /* the order the stages' waits count */
+#pragma unroll
+    for (int j = 0; j < 4; j++) sc[j] = srow[j][0];
+    asm volatile("" ::: "memory");
+    fetch(1u, 1u);
+    uint32_t slot = 0u;
+    /* stage s from `slot`; next: the codes of s + 1, refilled with s + 3 */
+    auto stage = [&](uint32_t s, u32x4_t &next, auto Odd) {
+        constexpr bool odd = decltype(Odd)::value;
+        /* younger than stage s's tokens: those of s + 1, a code load and four
+         * scales at least */
+        wait_vm<9>();
+        wait_lgkm<0>(); /* this wave's code writes */
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const uint32_t s1 = slot == 2u ? 0u : slot + 1u, s2 = slot == 0u ? 2u : slot - 1u;
+        fetch(s + 2u, s2);
+        if constexpr (odd) wait_vm<9>(); /* this block's scales: nine loads ago */
+        asm volatile("" ::: "memory");
+        const uint32_t st = (kWA + kWB) * slot;
+#pragma unroll
+        for (int ks = 0; ks < 2; ks++) {
+            u32x4_t af[4], bf[4];
+            const uint32_t o = st + (ks ? slot1 : slot0);
+            asm volatile(
+                "ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:2048\n\t"
+                "ds_read_b128 %2, %8 offset:4096\n\tds_read_b128 %3, %8 offset:6144\n\t"
+                "ds_read_b128 %4, %9\n\tds_read_b128 %5, %9 offset:2048\n\t"
+                "ds_read_b128 %6, %9 offset:4096\n\tds_read_b128 %7, %9 offset:6144\n\t"
+                "s_waitcnt lgkmcnt(0)"
+                : "=&v"(af[0]), "=&v"(af[1]), "=&v"(af[2]), "=&v"(af[3]), "=&v"(bf[0]),
+                  "=&v"(bf[1]), "=&v"(bf[2]), "=&v"(bf[3])
+                : "v"(a_base + o), "v"(b_base + o));
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const f32x4_t in = !odd && ks == 0 ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : blk[i][j];
+                    blk[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8_t, af[i]), __builtin_bit_cast(bf16x8_t, bf[j]), in,
+                        0, 0, 0);
+                }
+        }
+        /* used here and not before the products: the loads are still out */
+        asm volatile("" : "+v"(next) : : "memory");
+        write(next, s1);
+        next = codes(s + 3u);
+        slot = s1;
+        if constexpr (odd) { /* acc += scale x block sum; the next block's scales */
+            const uint32_t b = s / 2u + 1u < nblk ? s / 2u + 1u : s / 2u;
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(blk[i][j][r], sc[j], acc[i][j][r]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) sc[j] = srow[j][b];
+        }
+    };
+    for (uint32_t s = 0u; s < nsteps; s += 2u) { /* K % 128 == 0: an even count */
+        stage(s, q1, std::false_type{});
+        stage(s + 1u, q0, std::true_type{});
+    }
+    wait_vm<0>(); /* the loads past the end land before the LDS is given back */
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t n = n0 + 64u * wn + 16u * (uint32_t)j + c;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const uint32_t t = t0 + 64u * wm + 16u * (uint32_t)i + 4u * g + (uint32_t)r;
+                if (t < T && n < N) P.out[(uint64_t)t * N + n] = f32_to_bf16(acc[i][j][r]);
+            }
+        }
+}
+
 }  // namespace
 
 bool proj_mfma_supported(uint32_t tokens, uint32_t rows, uint32_t cols, bool q8,
@@ -236,8 +407,13 @@ bool proj_mfma_supported(uint32_t tokens, uint32_t rows, uint32_t cols, bool q8,
 bool launch_proj_mfma(uint16_t *out, const void *x, const void *weights, const float *scales,
                       uint32_t T, uint32_t N, uint32_t K, bool q8, hipStream_t st) {
     if (!proj_mfma_supported(T, N, K, q8, weights, x) || (q8 && !scales)) return false;
-    const uint32_t works = ((T + kPT - 1u) / kPT) * ((N + kPT - 1u) / kPT);
     const ProjArgs A{out, (const uint16_t *)x, weights, scales, T, N, K};
+    if (q8 && wide_pays(T, N) && ((uintptr_t)weights % 16u) == 0u) {
+        const uint32_t wide = ((T + kWT - 1u) / kWT) * ((N + kWN - 1u) / kWN);
+        hipLaunchKernelGGL(proj_wide_kernel, dim3(8u * ((wide + 7u) / 8u)), dim3(512), 0, st, A);
+        return hipGetLastError() == hipSuccess;
+    }
+    const uint32_t works = ((T + kPT - 1u) / kPT) * ((N + kPT - 1u) / kPT);
     const dim3 grid(8u * ((works + 7u) / 8u));
     if (q8)
         hipLaunchKernelGGL(HIP_KERNEL_NAME(proj_mfma_kernel<true>), grid, dim3(512), 0, st, A);

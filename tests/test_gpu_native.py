@@ -242,3 +242,13 @@ def test_proj_mfma_ragged_vs_row_kernels(cuda, q8, T, rows, cols):
     assert not lib().k3_moe_proj_mfma_bf16(P(got), P(wd), P(sd), P(xd), T, rows, cols - 32, q8, st)
     if q8:
         assert not lib().k3_moe_proj_mfma_bf16(P(got), P(wd), None, P(xd), T, rows, cols, q8, st)
+
+
+@pytest.mark.parametrize("T,rows,cols", [(32769, 128, 128), (1025, 4100, 256), (2055, 2100, 384),
+                                         (1279, 3201, 3584)])
+def test_proj_mfma_wide_tiles(cuda, T, rows, cols):
+    """The 256 x 128 tiles, taken where the 128 x 128 ones need more than one
+    round over the 256 compute units: one token and one row past a tile, one
+    to 28 scale blocks; the comparison and the bounds of the ragged test above."""
+    assert -(-T // 128) * -(-rows // 128) > 256 >= -(-T // 256) * -(-rows // 128)
+    test_proj_mfma_ragged_vs_row_kernels(cuda, True, T, rows, cols)
