@@ -13,13 +13,13 @@
  * groups and scale each): a tolerance of fp32 reassociation, far inside
  * one bf16 rounding of the output.
  *
- * Block tile 128 tokens x 128 rows, 8 waves of 32 x 64 (2 x 4
+ * bf16 weights: block tile 128 tokens x 128 rows, 8 waves of 32 x 64 (2 x 4
  * V_MFMA_F32_16X16X32_BF16 tiles), K steps of 64 through two LDS buffers
- * (rows padded to 144 bytes), global loads two steps ahead. Codes are
- * converted to bf16 on their way into LDS. A Q8-128 block is two K steps:
- * its four MFMAs per tile chain in a block sum that is then scaled into
- * the accumulator with one fma per output; the next block's scales are
- * loaded a block ahead. Tiles are dealt to the XCDs in contiguous ranges,
+ * (rows padded to 144 bytes), global loads two steps ahead. Codes: tiles of
+ * 64 x 64 to 256 x 128 fed by direct-to-LDS loads, chosen by the rounds they
+ * take (q8_tile); the four MFMAs of a 128-column block chain in a block sum
+ * that is then scaled into the accumulator with one fma per output, in every
+ * tile alike: the same bits. Tiles are dealt to the XCDs in contiguous ranges,
  * a token tile's row tiles together.
  */
 #include "k3_device.h"
@@ -36,6 +36,8 @@ namespace {
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4_a8_t __attribute__((ext_vector_type(4), aligned(8)));
 
 constexpr uint32_t kPT = 128, kPK = 64, kPPad = 144;
 
@@ -65,35 +67,24 @@ __device__ __forceinline__ uint4 codes_to_bf16(uint2 v) {
     return make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-/* The thread's two rows of one K step: x as 16 bytes, weights as 16
- * (bf16) or 8 (codes) bytes, converted to bf16 on the store. */
-template <bool Q8>
-using WeightPiece = typename std::conditional<Q8, uint2, uint4>::type;
-
-template <bool Q8>
-__device__ __forceinline__ void proj_load(uint4 &a0, uint4 &a1, WeightPiece<Q8> &b0,
-                                          WeightPiece<Q8> &b1, const uint8_t *xb,
-                                          const uint8_t *wb, uint32_t ao0, uint32_t ao1,
-                                          uint32_t bo0, uint32_t bo1, uint32_t s) {
-    const uint32_t ka = 2u * kPK * s, kw = (Q8 ? 1u : 2u) * kPK * s;
-    a0 = *(const uint4 *)(xb + ao0 + ka);
-    a1 = *(const uint4 *)(xb + ao1 + ka);
-    b0 = *(const WeightPiece<Q8> *)(wb + bo0 + kw);
-    b1 = *(const WeightPiece<Q8> *)(wb + bo1 + kw);
+/* The thread's two rows of one K step of x and of the weights. */
+__device__ __forceinline__ void proj_load(uint4 &a0, uint4 &a1, uint4 &b0, uint4 &b1,
+                                          const uint8_t *xb, const uint8_t *wb, uint32_t ao0,
+                                          uint32_t ao1, uint32_t bo0, uint32_t bo1, uint32_t s) {
+    const uint32_t k = 2u * kPK * s;
+    a0 = *(const uint4 *)(xb + ao0 + k);
+    a1 = *(const uint4 *)(xb + ao1 + k);
+    b0 = *(const uint4 *)(wb + bo0 + k);
+    b1 = *(const uint4 *)(wb + bo1 + k);
 }
 
-__device__ __forceinline__ uint4 as_bf16x8(uint2 codes) { return codes_to_bf16(codes); }
-__device__ __forceinline__ uint4 as_bf16x8(uint4 bf16) { return bf16; }
-
-template <bool Q8>
 __device__ __forceinline__ void proj_store(ProjStage &buf, uint32_t off, const uint4 &a0,
-                                           const uint4 &a1, const WeightPiece<Q8> &b0,
-                                           const WeightPiece<Q8> &b1) {
+                                           const uint4 &a1, const uint4 &b0, const uint4 &b1) {
     constexpr uint32_t R64 = 64u * kPPad;
     *(uint4 *)(buf[0] + off) = a0;
     *(uint4 *)(buf[0] + off + R64) = a1;
-    *(uint4 *)(buf[1] + off) = as_bf16x8(b0);
-    *(uint4 *)(buf[1] + off + R64) = as_bf16x8(b1);
+    *(uint4 *)(buf[1] + off) = b0;
+    *(uint4 *)(buf[1] + off + R64) = b1;
 }
 
 /* acc[i][j] += A(wave rows i) . B(wave rows j) over one K step. */
@@ -118,7 +109,6 @@ __device__ __forceinline__ void proj_compute(f32x4_t (&acc)[2][4], const ProjSta
     }
 }
 
-template <bool Q8>
 __global__ __launch_bounds__(512) void proj_mfma_kernel(ProjArgs P) {
     __shared__ __attribute__((aligned(16))) ProjStage lds[2];
     const uint32_t T = P.T, N = P.N, K = P.K;
@@ -132,84 +122,43 @@ __global__ __launch_bounds__(512) void proj_mfma_kernel(ProjArgs P) {
     /* thread tid loads piece tid % 8 (8 columns) of rows tid / 8 and tid /
      * 8 + 64; rows past T or N clamp to the last one (not stored) */
     const uint32_t r0 = tid >> 3, pc = tid & 7u;
-    constexpr uint32_t wbytes = Q8 ? 1u : 2u;
     uint32_t ao[2], bo[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) {
         const uint32_t ta = t0 + r0 + 64u * i, nb = n0 + r0 + 64u * i;
         ao[i] = ((ta < T ? ta : T - 1u) * K + 8u * pc) * 2u;
-        bo[i] = ((nb < N ? nb : N - 1u) * K + 8u * pc) * wbytes;
+        bo[i] = ((nb < N ? nb : N - 1u) * K + 8u * pc) * 2u;
     }
     const uint8_t *xb = (const uint8_t *)P.x, *wb = (const uint8_t *)P.w;
     const uint32_t soff = r0 * kPPad + 16u * pc;
     const uint32_t a_off = (32u * wm + c) * kPPad + 16u * g;
     const uint32_t b_off = (64u * wn + c) * kPPad + 16u * g;
-    /* Q8: the scales of this lane's four weight rows (one per n-tile) */
-    const uint32_t nblk = K / 128u;
-    const float *srow[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const uint32_t r = n0 + 64u * wn + 16u * (uint32_t)j + c;
-        srow[j] = P.scales + (uint64_t)(r < N ? r : N - 1u) * nblk;
-    }
-    f32x4_t acc[2][4], blk[2][4];
+    f32x4_t acc[2][4];
 #pragma unroll
     for (int i = 0; i < 2; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            blk[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-    float sc[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-    if constexpr (Q8) {
-#pragma unroll
-        for (int j = 0; j < 4; j++) sc[j] = srow[j][0];
-    }
+        for (int j = 0; j < 4; j++) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t nsteps = K / kPK, last = nsteps - 1u;
     /* two register sets: step s + 2's loads are issued at the start of
      * step s; loads and stores are unconditional (steps past the end
      * reload the last one into a buffer nobody reads) */
-    uint4 a0, a1, p0, p1;
-    WeightPiece<Q8> b0, b1, q0, q1;
-    proj_load<Q8>(a0, a1, b0, b1, xb, wb, ao[0], ao[1], bo[0], bo[1], 0u);
-    proj_load<Q8>(p0, p1, q0, q1, xb, wb, ao[0], ao[1], bo[0], bo[1], 1u < last ? 1u : last);
-    proj_store<Q8>(lds[0], soff, a0, a1, b0, b1);
+    uint4 a0, a1, b0, b1, p0, p1, q0, q1;
+    proj_load(a0, a1, b0, b1, xb, wb, ao[0], ao[1], bo[0], bo[1], 0u);
+    proj_load(p0, p1, q0, q1, xb, wb, ao[0], ao[1], bo[0], bo[1], 1u < last ? 1u : last);
+    proj_store(lds[0], soff, a0, a1, b0, b1);
     __syncthreads();
     for (uint32_t s = 0; s < nsteps; s += 2u) {
-        /* Q8: steps s, s + 1 are 128-column block s / 2 (K % 128 == 0);
-         * the next block's scales load during this block's two steps */
-        float nx[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-        if constexpr (Q8) {
-            const uint32_t b1 = s / 2u + 1u < nblk ? s / 2u + 1u : s / 2u;
-#pragma unroll
-            for (int j = 0; j < 4; j++) nx[j] = srow[j][b1];
-        }
-        proj_load<Q8>(a0, a1, b0, b1, xb, wb, ao[0], ao[1], bo[0], bo[1],
+        proj_load(a0, a1, b0, b1, xb, wb, ao[0], ao[1], bo[0], bo[1],
                       s + 2u < last ? s + 2u : last);
-        if constexpr (Q8) proj_compute(blk, lds[0], a_off, b_off);
-        else proj_compute(acc, lds[0], a_off, b_off);
-        proj_store<Q8>(lds[1], soff, p0, p1, q0, q1);
+        proj_compute(acc, lds[0], a_off, b_off);
+        proj_store(lds[1], soff, p0, p1, q0, q1);
         __syncthreads();
         if (s + 1u < nsteps) {
-            proj_load<Q8>(p0, p1, q0, q1, xb, wb, ao[0], ao[1], bo[0], bo[1],
-                          s + 3u < last ? s + 3u : last);
-            if constexpr (Q8) proj_compute(blk, lds[1], a_off, b_off);
-            else proj_compute(acc, lds[1], a_off, b_off);
-            proj_store<Q8>(lds[0], soff, a0, a1, b0, b1);
+            proj_load(p0, p1, q0, q1, xb, wb, ao[0], ao[1], bo[0], bo[1],
+                      s + 3u < last ? s + 3u : last);
+            proj_compute(acc, lds[1], a_off, b_off);
+            proj_store(lds[0], soff, a0, a1, b0, b1);
             __syncthreads();
-        }
-        if constexpr (Q8) {
-            /* acc += scale * block sum */
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(blk[i][j][r], sc[j], acc[i][j][r]);
-                    blk[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-                }
-#pragma unroll
-            for (int j = 0; j < 4; j++) sc[j] = nx[j];
         }
     }
 #pragma unroll
@@ -239,16 +188,6 @@ __global__ __launch_bounds__(512) void proj_mfma_kernel(ProjArgs P) {
  */
 constexpr uint32_t kWT = 256, kWN = 128;              /* block tile */
 constexpr uint32_t kWA = kWT * 128u, kWB = kWN * 128u; /* bytes of a stage */
-
-/* Both kernels hold one block a CU, and a round of tiles over the 256 CUs
- * takes the wide one 6/5 as long for twice the work (7168 columns: 123 and
- * 103 us, 1024 columns: 21 and 17 us): wide where that pays for its rounds. */
-static bool wide_pays(uint32_t T, uint32_t N) {
-    auto rounds = [&](uint32_t tt) {
-        return ((T + tt - 1u) / tt * (uint64_t)((N + 127u) / 128u) + 255u) / 256u;
-    };
-    return 6u * rounds(kWT) < 5u * rounds(kPT);
-}
 
 __global__ __launch_bounds__(512, 2) void proj_wide_kernel(ProjArgs P) {
     __shared__ __attribute__((aligned(16))) uint8_t smem[3u * (kWA + kWB)];
@@ -292,7 +231,7 @@ __global__ __launch_bounds__(512, 2) void proj_wide_kernel(ProjArgs P) {
                 (lds_void *)(uintptr_t)(lds + (kWA + kWB) * slot + 4096u * wave + 1024u * m), 16, 0,
                 0);
     };
-    auto codes = [&](uint32_t s) { return *(const u32x4_t *)(ws + kPK * (s < last ? s : last)); };
+    auto codes = [&](uint32_t s) { return (u32x4_t) * (const u32x4_a8_t *)(ws + kPK * (s < last ? s : last)); };
     auto write = [&](const u32x4_t &q, uint32_t slot) {
         const uint32_t base = lds + (kWA + kWB) * slot;
         const uint4 lo = codes_to_bf16(make_uint2(q[0], q[1])), hi = codes_to_bf16(make_uint2(q[2], q[3]));
@@ -394,6 +333,241 @@ __global__ __launch_bounds__(512, 2) void proj_wide_kernel(ProjArgs P) {
         }
 }
 
+/*
+ * The Q8-128 form for fewer tokens: 16 WT WM tokens x 16 NR WN rows of eight
+ * waves, everything by direct-to-LDS loads into a ring of RING stages of one
+ * scale block (128 columns: tokens as bf16, codes as bytes, each wave's
+ * scales), explicit LDS accesses and waits as above. Codes become bf16 after
+ * their LDS read. A stage is LDS reads, then conversions and MFMAs, with one
+ * barrier; the LDS reads bound the larger tiles (a 64-row wave reads every
+ * token of the block), the latency of a stage the smallest. A 128 x 128 tile
+ * staged through registers two steps ahead took 103 us for 7168 columns at any
+ * token count up to a round. Before -> after, us: 6144 x 7168, 96 tokens 102
+ * -> 36, 300 tokens 103 -> 54, 512 tokens 104 -> 74, 1024 tokens 204 (127 on
+ * the tile above) -> 127; 7168 x 3584, 96 tokens 51 -> 19; 1024 x 1024, 96
+ * tokens 17 -> 7.7.
+ */
+/* The fragments of two 32-column steps, and of a stage where they fit, each
+ * read by one statement that waits for them. */
+template <int WT, int NR>
+struct RingFrags {
+    u32x4_t a[2][WT];
+    u32x2_t b[2][NR];
+};
+__device__ __forceinline__ void ring_read(RingFrags<4, 2> &f, uint32_t a0, uint32_t a1, uint32_t b0,
+                                          uint32_t b1) {
+    asm volatile(
+        "ds_read_b128 %0, %12\n\tds_read_b128 %1, %12 offset:2048\n\t"
+        "ds_read_b128 %2, %12 offset:4096\n\tds_read_b128 %3, %12 offset:6144\n\t"
+        "ds_read_b64 %8, %14\n\tds_read_b64 %9, %14 offset:2048\n\t"
+        "ds_read_b128 %4, %13\n\tds_read_b128 %5, %13 offset:2048\n\t"
+        "ds_read_b128 %6, %13 offset:4096\n\tds_read_b128 %7, %13 offset:6144\n\t"
+        "ds_read_b64 %10, %15\n\tds_read_b64 %11, %15 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+        : "=&v"(f.a[0][0]), "=&v"(f.a[0][1]), "=&v"(f.a[0][2]), "=&v"(f.a[0][3]), "=&v"(f.a[1][0]),
+          "=&v"(f.a[1][1]), "=&v"(f.a[1][2]), "=&v"(f.a[1][3]), "=&v"(f.b[0][0]), "=&v"(f.b[0][1]),
+          "=&v"(f.b[1][0]), "=&v"(f.b[1][1])
+        : "v"(a0), "v"(a1), "v"(b0), "v"(b1)
+        : "memory");
+}
+
+
+template <uint32_t H> /* bytes between the two halves of the tokens */
+__device__ __forceinline__ void ring_read(RingFrags<2, 1> (&f)[2], const uint32_t (&a)[2],
+                                          const uint32_t (&b)[4]) {
+    asm volatile(
+        "ds_read_b128 %0, %12\n\tds_read_b128 %1, %12 offset:2048\n\tds_read_b64 %8, %14\n\t"
+        "ds_read_b128 %2, %13\n\tds_read_b128 %3, %13 offset:2048\n\tds_read_b64 %9, %15\n\t"
+        "ds_read_b128 %4, %12 offset:%18\n\tds_read_b128 %5, %12 offset:%19\n\tds_read_b64 %10, %16\n\t"
+        "ds_read_b128 %6, %13 offset:%18\n\tds_read_b128 %7, %13 offset:%19\n\tds_read_b64 %11, %17\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(f[0].a[0][0]), "=&v"(f[0].a[0][1]), "=&v"(f[0].a[1][0]), "=&v"(f[0].a[1][1]),
+          "=&v"(f[1].a[0][0]), "=&v"(f[1].a[0][1]), "=&v"(f[1].a[1][0]), "=&v"(f[1].a[1][1]),
+          "=&v"(f[0].b[0][0]), "=&v"(f[0].b[1][0]), "=&v"(f[1].b[0][0]), "=&v"(f[1].b[1][0])
+        : "v"(a[0]), "v"(a[1]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "i"(H), "i"(H + 2048u)
+        : "memory");
+}
+template <uint32_t H>
+__device__ __forceinline__ void ring_read(RingFrags<2, 2> (&f)[2], const uint32_t (&a)[2],
+                                          const uint32_t (&b)[4]) {
+    asm volatile(
+        "ds_read_b128 %0, %16\n\tds_read_b128 %1, %16 offset:2048\n\t"
+        "ds_read_b64 %8, %18\n\tds_read_b64 %9, %18 offset:2048\n\t"
+        "ds_read_b128 %2, %17\n\tds_read_b128 %3, %17 offset:2048\n\t"
+        "ds_read_b64 %10, %19\n\tds_read_b64 %11, %19 offset:2048\n\t"
+        "ds_read_b128 %4, %16 offset:%22\n\tds_read_b128 %5, %16 offset:%23\n\t"
+        "ds_read_b64 %12, %20\n\tds_read_b64 %13, %20 offset:2048\n\t"
+        "ds_read_b128 %6, %17 offset:%22\n\tds_read_b128 %7, %17 offset:%23\n\t"
+        "ds_read_b64 %14, %21\n\tds_read_b64 %15, %21 offset:2048\n\t"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(f[0].a[0][0]), "=&v"(f[0].a[0][1]), "=&v"(f[0].a[1][0]), "=&v"(f[0].a[1][1]),
+          "=&v"(f[1].a[0][0]), "=&v"(f[1].a[0][1]), "=&v"(f[1].a[1][0]), "=&v"(f[1].a[1][1]),
+          "=&v"(f[0].b[0][0]), "=&v"(f[0].b[0][1]), "=&v"(f[0].b[1][0]), "=&v"(f[0].b[1][1]),
+          "=&v"(f[1].b[0][0]), "=&v"(f[1].b[0][1]), "=&v"(f[1].b[1][0]), "=&v"(f[1].b[1][1])
+        : "v"(a[0]), "v"(a[1]), "v"(b[0]), "v"(b[1]), "v"(b[2]), "v"(b[3]), "i"(H), "i"(H + 2048u)
+        : "memory");
+}
+
+template <int WT, int NR, int WM, int RING>
+struct Ring {
+    static constexpr uint32_t WN = 8 / WM, TT = 16 * WT * WM, TN = 16 * NR * WN;
+    static constexpr uint32_t A = 256u * TT, B = 128u * TN, S = 2048u; /* bytes of a stage */
+    static constexpr uint32_t STAGE = A + B + S;
+    static constexpr int DA = TT / 32, DB = TN / 64, D = DA + DB + 1; /* loads a wave and stage */
+    static_assert(RING * STAGE <= 160u * 1024u, "LDS");
+};
+
+template <int WT, int NR, int WM, int RING>
+__global__ __launch_bounds__(512) void proj_ring_kernel(ProjArgs P) {
+    using C = Ring<WT, NR, WM, RING>;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[RING * C::STAGE];
+    const uint32_t T = P.T, N = P.N, K = P.K;
+    const uint32_t ntt = (T + C::TT - 1u) / C::TT, nnt = (N + C::TN - 1u) / C::TN;
+    const uint32_t works = ntt * nnt, per = (works + 7u) / 8u;
+    const uint32_t j8 = blockIdx.x >> 3, wk = (blockIdx.x & 7u) * per + j8;
+    if (j8 >= per || wk >= works) return;
+    const uint32_t t0 = (wk / nnt) * C::TT, n0 = (wk % nnt) * C::TN;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t wm = wave / C::WN, wn = wave % C::WN, g = lane >> 4, c = lane & 15u;
+    const uint32_t lds = lds_addr(smem);
+    /* 1 KB chunks (8 rows x 128 bytes) of each wave: tokens [64 columns][16
+     * rows][8 rows], codes [16 rows][8 rows]; rows past T or N repeat the
+     * last one (not stored) */
+    const uint8_t *xs[C::DA], *ws[C::DB];
+#pragma unroll
+    for (int m = 0; m < C::DA; m++) {
+        const uint32_t q = C::DA * wave + (uint32_t)m, h = q & 1u, col = q / (C::TT / 8u);
+        const uint32_t r = t0 + 16u * (q % (C::TT / 8u) >> 1) + a_dma_row(lane, h);
+        xs[m] = (const uint8_t *)P.x + 2ull * (r < T ? r : T - 1u) * K + 128u * col + 16u * a_dma_piece(lane, h);
+    }
+#pragma unroll
+    for (int m = 0; m < C::DB; m++) {
+        const uint32_t q = C::DB * wave + (uint32_t)m, h = q & 1u;
+        const uint32_t r = n0 + 16u * (q >> 1) + a_dma_row(lane, h);
+        ws[m] = (const uint8_t *)P.w + (uint64_t)(r < N ? r : N - 1u) * K + 16u * a_dma_piece(lane, h);
+    }
+    const uint32_t nblk = K / 128u, last = nblk - 1u;
+    const uint32_t sr = n0 + 16u * NR * wn + (lane & (16u * NR - 1u));
+    const float *sp = P.scales + (uint64_t)(sr < N ? sr : N - 1u) * nblk;
+    auto fetch = [&](uint32_t s, uint32_t base) { /* past the end: the last stage again */
+        const uint32_t b = s < last ? s : last;
+#pragma unroll
+        for (int m = 0; m < C::DB; m++)
+            __builtin_amdgcn_global_load_lds((const void *)(ws[m] + 128u * b),
+                                             (lds_void *)(uintptr_t)(base + C::A + 1024u * (C::DB * wave + m)),
+                                             16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void *)(sp + b),
+                                         (lds_void *)(uintptr_t)(base + C::A + C::B + 256u * wave), 4, 0, 0);
+#pragma unroll
+        for (int m = 0; m < C::DA; m++)
+            __builtin_amdgcn_global_load_lds((const void *)(xs[m] + 256u * b),
+                                             (lds_void *)(uintptr_t)(base + 1024u * (C::DA * wave + m)), 16,
+                                             0, 0);
+    };
+    f32x4_t acc[WT][NR];
+#pragma unroll
+    for (int i = 0; i < WT; i++)
+#pragma unroll
+        for (int j = 0; j < NR; j++) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const uint32_t a_base = 2048u * WT * wm, b_base = C::A + 2048u * NR * wn;
+    const uint32_t aslot[2] = {a_base + a_slot(c, g), a_base + a_slot(c, 4u + g)};
+    uint32_t bslot[4];
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; k++) bslot[k] = b_base + a_slot(c, 2u * k + (g >> 1)) + 8u * (g & 1u);
+    const uint32_t s_slot = C::A + C::B + 256u * wave + 4u * c;
+#pragma unroll
+    for (uint32_t s = 0; s < RING - 1u; s++) fetch(s, lds + C::STAGE * s);
+    uint32_t cur = lds, free_ = lds + C::STAGE * (RING - 1u);
+    const uint32_t end = lds + C::STAGE * RING;
+    for (uint32_t s = 0; s < nblk; s++) {
+        wait_vm<C::D *(RING - 2)>(); /* this wave's loads of stage s */
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        fetch(s + RING - 1u, free_);
+        f32x4_t blk[WT][NR];
+        float sc[NR];
+        if constexpr (NR == 1)
+            asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=&v"(sc[0]) : "v"(cur + s_slot) : "memory");
+        else
+            asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %2 offset:64\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(sc[0]), "=&v"(sc[1])
+                         : "v"(cur + s_slot)
+                         : "memory");
+        const uint32_t as[2] = {cur + aslot[0], cur + aslot[1]};
+        const uint32_t bs[4] = {cur + bslot[0], cur + bslot[1], cur + bslot[2], cur + bslot[3]};
+        RingFrags<WT, NR> fr[2];
+        if constexpr (WT == 2) ring_read<128u * C::TT>(fr, as, bs);
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            RingFrags<WT, NR> &f = fr[h];
+            if constexpr (WT == 4)
+                ring_read(f, as[0] + 128u * C::TT * h, as[1] + 128u * C::TT * h, bs[2 * h], bs[2 * h + 1]);
+#pragma unroll
+            for (int ks = 0; ks < 2; ks++)
+#pragma unroll
+                for (int j = 0; j < NR; j++) {
+                    const bf16x8_t b = __builtin_bit_cast(
+                        bf16x8_t, codes_to_bf16(make_uint2(f.b[ks][j][0], f.b[ks][j][1])));
+#pragma unroll
+                    for (int i = 0; i < WT; i++)
+                        blk[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                            __builtin_bit_cast(bf16x8_t, f.a[ks][i]), b,
+                            h == 0 && ks == 0 ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : blk[i][j], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < WT; i++)
+#pragma unroll
+            for (int j = 0; j < NR; j++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(blk[i][j][r], sc[j], acc[i][j][r]);
+        free_ = cur;
+        cur += C::STAGE;
+        if (cur == end) cur = lds;
+    }
+    wait_vm<0>(); /* the loads past the end land before the LDS is given back */
+#pragma unroll
+    for (int i = 0; i < WT; i++)
+#pragma unroll
+        for (int j = 0; j < NR; j++) {
+            const uint32_t n = n0 + 16u * (NR * wn + (uint32_t)j) + c;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const uint32_t t = t0 + 16u * (WT * wm + (uint32_t)i) + 4u * g + (uint32_t)r;
+                if (t < T && n < N) P.out[(uint64_t)t * N + n] = f32_to_bf16(acc[i][j][r]);
+            }
+        }
+}
+
+template <int WT, int NR, int WM, int RING>
+bool launch_ring(const ProjArgs &A, hipStream_t st) {
+    using C = Ring<WT, NR, WM, RING>;
+    const uint32_t works = ((A.T + C::TT - 1u) / C::TT) * ((A.N + C::TN - 1u) / C::TN);
+    hipLaunchKernelGGL(HIP_KERNEL_NAME(proj_ring_kernel<WT, NR, WM, RING>),
+                       dim3(8u * ((works + 7u) / 8u)), dim3(512), 0, st, A);
+    return hipGetLastError() == hipSuccess;
+}
+
+/* Every Q8 tile holds one block a CU, so a call takes its rounds of tiles over
+ * the 256 CUs times a round: 64 x 64 tokens x rows 35 us of 7168 columns, 64 x
+ * 128 52, 128 x 128 72 and 256 x 128 124. The cheapest, the larger tile of
+ * equals. (6144 x 7168, the four in turn, us: 96 tokens 36 53 71 123, 256
+ * tokens 70 56 73 124, 512 tokens 101 105 74 124, 1280 tokens 262 211 151 130,
+ * 8192 tokens 1600 1270 930 796.) */
+int q8_tile(uint32_t T, uint32_t N) {
+    static constexpr uint32_t tt[4] = {64u, 64u, 128u, 256u}, tn[4] = {64u, 128u, 128u, 128u};
+    static constexpr uint32_t cost[4] = {10u, 15u, 20u, 35u};
+    int best = 0;
+    uint64_t least = ~0ull;
+    for (int i = 0; i < 4; i++) {
+        const uint64_t works = (uint64_t)((T + tt[i] - 1u) / tt[i]) * ((N + tn[i] - 1u) / tn[i]);
+        const uint64_t t = (works + 255u) / 256u * cost[i];
+        if (t <= least) least = t, best = i;
+    }
+    return best;
+}
+
 }  // namespace
 
 bool proj_mfma_supported(uint32_t tokens, uint32_t rows, uint32_t cols, bool q8,
@@ -408,17 +582,18 @@ bool launch_proj_mfma(uint16_t *out, const void *x, const void *weights, const f
                       uint32_t T, uint32_t N, uint32_t K, bool q8, hipStream_t st) {
     if (!proj_mfma_supported(T, N, K, q8, weights, x) || (q8 && !scales)) return false;
     const ProjArgs A{out, (const uint16_t *)x, weights, scales, T, N, K};
-    if (q8 && wide_pays(T, N) && ((uintptr_t)weights % 16u) == 0u) {
-        const uint32_t wide = ((T + kWT - 1u) / kWT) * ((N + kWN - 1u) / kWN);
-        hipLaunchKernelGGL(proj_wide_kernel, dim3(8u * ((wide + 7u) / 8u)), dim3(512), 0, st, A);
+    if (q8) {
+        switch (q8_tile(T, N)) {
+        case 0: return launch_ring<2, 1, 2, 6>(A, st);
+        case 1: return launch_ring<2, 2, 2, 4>(A, st);
+        case 2: return launch_ring<4, 2, 2, 3>(A, st);
+        }
+        const uint32_t works = ((T + kWT - 1u) / kWT) * ((N + kWN - 1u) / kWN);
+        hipLaunchKernelGGL(proj_wide_kernel, dim3(8u * ((works + 7u) / 8u)), dim3(512), 0, st, A);
         return hipGetLastError() == hipSuccess;
     }
     const uint32_t works = ((T + kPT - 1u) / kPT) * ((N + kPT - 1u) / kPT);
-    const dim3 grid(8u * ((works + 7u) / 8u));
-    if (q8)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(proj_mfma_kernel<true>), grid, dim3(512), 0, st, A);
-    else
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(proj_mfma_kernel<false>), grid, dim3(512), 0, st, A);
+    hipLaunchKernelGGL(proj_mfma_kernel, dim3(8u * ((works + 7u) / 8u)), dim3(512), 0, st, A);
     return hipGetLastError() == hipSuccess;
 }
 

@@ -244,11 +244,13 @@ def test_proj_mfma_ragged_vs_row_kernels(cuda, q8, T, rows, cols):
         assert not lib().k3_moe_proj_mfma_bf16(P(got), P(wd), None, P(xd), T, rows, cols, q8, st)
 
 
-@pytest.mark.parametrize("T,rows,cols", [(32769, 128, 128), (1025, 4100, 256), (2055, 2100, 384),
-                                         (1279, 3201, 3584)])
-def test_proj_mfma_wide_tiles(cuda, T, rows, cols):
-    """The 256 x 128 tiles, taken where the 128 x 128 ones need more than one
-    round over the 256 compute units: one token and one row past a tile, one
-    to 28 scale blocks; the comparison and the bounds of the ragged test above."""
-    assert -(-T // 128) * -(-rows // 128) > 256 >= -(-T // 256) * -(-rows // 128)
+@pytest.mark.parametrize("T,rows,cols", [
+    (65, 129, 128), (1, 65, 3584), (300, 577, 768), (129, 200, 896),      # 64 x 64 tiles
+    (1000, 1030, 128), (961, 1025, 640),                                  # 64 x 128
+    (2000, 1090, 128), (1921, 1153, 512),                                 # 128 x 128
+    (32769, 128, 128), (1025, 4100, 256), (2055, 2100, 384), (1279, 3201, 3584)])  # 256 x 128
+def test_proj_mfma_q8_tiles(cuda, T, rows, cols):
+    """Every tile of the Q8 projections where its rounds make it the choice:
+    one token and one row past a tile, fewer scale blocks than a ring's
+    stages and more; the comparison and the bounds of the ragged test above."""
     test_proj_mfma_ragged_vs_row_kernels(cuda, True, T, rows, cols)
