@@ -338,14 +338,20 @@ __global__ __launch_bounds__(512, 2) void proj_wide_kernel(ProjArgs P) {
  * waves, everything by direct-to-LDS loads into a ring of RING stages of one
  * scale block (128 columns: tokens as bf16, codes as bytes, each wave's
  * scales), explicit LDS accesses and waits as above. Codes become bf16 after
- * their LDS read. A stage is LDS reads, then conversions and MFMAs, with one
- * barrier; the LDS reads bound the larger tiles (a 64-row wave reads every
- * token of the block), the latency of a stage the smallest. A 128 x 128 tile
- * staged through registers two steps ahead took 103 us for 7168 columns at any
- * token count up to a round. Before -> after, us: 6144 x 7168, 96 tokens 102
- * -> 36, 300 tokens 103 -> 54, 512 tokens 104 -> 74, 1024 tokens 204 (127 on
- * the tile above) -> 127; 7168 x 3584, 96 tokens 51 -> 19; 1024 x 1024, 96
- * tokens 17 -> 7.7.
+ * their LDS read. A stage is LDS reads (12 to 20 KB a wave), then conversions
+ * and MFMAs. With two row subtiles a wave the two waves of a SIMD take turns:
+ * waves 4..7 run one barrier behind, so one half reads while the other
+ * multiplies (64 x 128 tiles, 7168 columns: 53 -> 43 us a round, 128 x 128 72
+ * -> 70; with conversions and scaling in the reading phase 59 and 83; 64 x 64
+ * tiles 36 either way, 1024 columns 7.8 and 8.2; the 256 x 128 tiles above 124
+ * either way, 3584 columns 62 and 65). Conversions (1.5 instructions a code,
+ * once per token half) and MFMAs share the SIMD's issue: without any load in
+ * the loop a round still takes 29, 38 and 55 us. A 128 x 128 tile staged
+ * through registers two steps ahead took 103 us for 7168 columns at any token
+ * count up to a round. Before -> after, us: 6144 x 7168, 96 tokens 102 -> 36,
+ * 300 tokens 103 -> 45, 512 tokens 104 -> 72, 1536 tokens 305 (248 on the tile
+ * above) -> 211; 7168 x 3584, 96 tokens 51 -> 19; 1024 x 1024, 96 tokens 17 ->
+ * 7.8.
  */
 /* The fragments of two 32-column steps, and of a stage where they fit, each
  * read by one statement that waits for them. */
@@ -407,12 +413,23 @@ __device__ __forceinline__ void ring_read(RingFrags<2, 2> (&f)[2], const uint32_
         : "memory");
 }
 
+/* Between two phases of the alternating form. */
+__device__ __forceinline__ void phase_barrier() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int WT, int NR, int WM, int RING>
 struct Ring {
     static constexpr uint32_t WN = 8 / WM, TT = 16 * WT * WM, TN = 16 * NR * WN;
     static constexpr uint32_t A = 256u * TT, B = 128u * TN, S = 2048u; /* bytes of a stage */
     static constexpr uint32_t STAGE = A + B + S;
     static constexpr int DA = TT / 32, DB = TN / 64, D = DA + DB + 1; /* loads a wave and stage */
+    static constexpr bool ALT = NR == 2; /* the halves of the block alternate */
+    static_assert(WT == 2 || ALT, "four token subtiles read by halves of a stage");
     static_assert(RING * STAGE <= 160u * 1024u, "LDS");
 };
 
@@ -479,12 +496,19 @@ __global__ __launch_bounds__(512) void proj_ring_kernel(ProjArgs P) {
     for (uint32_t s = 0; s < RING - 1u; s++) fetch(s, lds + C::STAGE * s);
     uint32_t cur = lds, free_ = lds + C::STAGE * (RING - 1u);
     const uint32_t end = lds + C::STAGE * RING;
+    if constexpr (C::ALT) {
+        wait_vm<C::D *(RING - 2)>(); /* stage 0 */
+        phase_barrier();
+        if (wave >= 4u) phase_barrier();
+    }
     for (uint32_t s = 0; s < nblk; s++) {
-        wait_vm<C::D *(RING - 2)>(); /* this wave's loads of stage s */
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        fetch(s + RING - 1u, free_);
+        if constexpr (!C::ALT) {
+            wait_vm<C::D *(RING - 2)>(); /* this wave's loads of stage s */
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        }
+        fetch(s + RING - 1u, free_); /* stage s - 1's slot: every wave has read it */
         f32x4_t blk[WT][NR];
         float sc[NR];
         if constexpr (NR == 1)
@@ -497,12 +521,21 @@ __global__ __launch_bounds__(512) void proj_ring_kernel(ProjArgs P) {
         const uint32_t as[2] = {cur + aslot[0], cur + aslot[1]};
         const uint32_t bs[4] = {cur + bslot[0], cur + bslot[1], cur + bslot[2], cur + bslot[3]};
         RingFrags<WT, NR> fr[2];
-        if constexpr (WT == 2) ring_read<128u * C::TT>(fr, as, bs);
+        if constexpr (WT == 2) {
+            ring_read<128u * C::TT>(fr, as, bs);
+            if constexpr (C::ALT) {
+                wait_vm<C::D *(RING - 2)>(); /* this wave's loads of stage s + 1 */
+                phase_barrier();
+            }
+        }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             RingFrags<WT, NR> &f = fr[h];
-            if constexpr (WT == 4)
+            if constexpr (WT == 4) {
                 ring_read(f, as[0] + 128u * C::TT * h, as[1] + 128u * C::TT * h, bs[2 * h], bs[2 * h + 1]);
+                if (h == 1) wait_vm<C::D *(RING - 2)>();
+                phase_barrier();
+            }
 #pragma unroll
             for (int ks = 0; ks < 2; ks++)
 #pragma unroll
@@ -515,6 +548,7 @@ __global__ __launch_bounds__(512) void proj_ring_kernel(ProjArgs P) {
                             __builtin_bit_cast(bf16x8_t, f.a[ks][i]), b,
                             h == 0 && ks == 0 ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : blk[i][j], 0, 0, 0);
                 }
+            if (WT == 4 && h == 0) phase_barrier();
         }
 #pragma unroll
         for (int i = 0; i < WT; i++)
@@ -522,9 +556,13 @@ __global__ __launch_bounds__(512) void proj_ring_kernel(ProjArgs P) {
             for (int j = 0; j < NR; j++)
 #pragma unroll
                 for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(blk[i][j][r], sc[j], acc[i][j][r]);
+        if constexpr (C::ALT) phase_barrier();
         free_ = cur;
         cur += C::STAGE;
         if (cur == end) cur = lds;
+    }
+    if constexpr (C::ALT) {
+        if (wave < 4u) phase_barrier();
     }
     wait_vm<0>(); /* the loads past the end land before the LDS is given back */
 #pragma unroll
@@ -550,14 +588,15 @@ bool launch_ring(const ProjArgs &A, hipStream_t st) {
 }
 
 /* Every Q8 tile holds one block a CU, so a call takes its rounds of tiles over
- * the 256 CUs times a round: 64 x 64 tokens x rows 35 us of 7168 columns, 64 x
- * 128 52, 128 x 128 72 and 256 x 128 124. The cheapest, the larger tile of
- * equals. (6144 x 7168, the four in turn, us: 96 tokens 36 53 71 123, 256
- * tokens 70 56 73 124, 512 tokens 101 105 74 124, 1280 tokens 262 211 151 130,
- * 8192 tokens 1600 1270 930 796.) */
+ * the 256 CUs times a round: 64 x 64 tokens x rows 36 us of 7168 columns, 64 x
+ * 128 43, 128 x 128 71 and 256 x 128 124. The cheapest, the larger tile of
+ * equals. (6144 x 7168, us: 300 tokens 45 on 64 x 128, 68 on 64 x 64; 512
+ * tokens 72 on 128 x 128, 101 on 64 x 64; 1280 tokens 129 on 256 x 128, 151 on
+ * 128 x 128; 1536 tokens 211 on 128 x 128, 248 on 256 x 128.)
+ */
 int q8_tile(uint32_t T, uint32_t N) {
     static constexpr uint32_t tt[4] = {64u, 64u, 128u, 256u}, tn[4] = {64u, 128u, 128u, 128u};
-    static constexpr uint32_t cost[4] = {10u, 15u, 20u, 35u};
+    static constexpr uint32_t cost[4] = {10u, 12u, 20u, 35u};
     int best = 0;
     uint64_t least = ~0ull;
     for (int i = 0; i < 4; i++) {
