@@ -254,3 +254,25 @@ def test_proj_mfma_q8_tiles(cuda, T, rows, cols):
     one token and one row past a tile, fewer scale blocks than a ring's
     stages and more; the comparison and the bounds of the ragged test above."""
     test_proj_mfma_ragged_vs_row_kernels(cuda, True, T, rows, cols)
+
+
+@pytest.mark.parametrize("T,rows,cols", [(65, 129, 384), (961, 1025, 128), (1921, 1153, 128),
+                                         (1025, 4100, 256)])
+def test_proj_mfma_q8_codes_at_8_mod_16(cuda, T, rows, cols):
+    """Each tile with the codes at 8 mod 16: the bits of the aligned call."""
+    import ctypes
+    from moonshine_amd._lib import lib
+    g = torch.Generator().manual_seed(T + rows)
+    x = torch.randn((T, cols), generator=g).to(torch.bfloat16).to(cuda)
+    q = torch.randint(-127, 128, (rows * cols,), generator=g, dtype=torch.int8).to(cuda)
+    s = torch.rand((rows, cols // 128), generator=g).to(cuda)
+    shifted = torch.zeros(rows * cols + 16, dtype=torch.int8, device=cuda)
+    shifted[8:8 + rows * cols] = q
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    out = [torch.zeros((T, rows), dtype=torch.bfloat16, device=cuda) for _ in range(2)]
+    assert q.data_ptr() % 16 == 0 and shifted.data_ptr() % 16 == 0
+    for o, w in zip(out, (q, shifted[8:])):
+        assert lib().k3_moe_proj_mfma_bf16(P(o), P(w), P(s), P(x), T, rows, cols, True, st)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
