@@ -253,18 +253,22 @@ __global__ __launch_bounds__(512, 2) void proj_wide_kernel(ProjArgs P) {
     write(q0, 0u);
     asm volatile("" : "+v"(q1) : : "memory");
     fetch(0u, 0u);
+    fetch(1u, 1u);
     asm volatile("" ::: "memory");
     q0 = codes(2u); /* the order the stages' waits count */
 #pragma unroll
     for (int j = 0; j < 4; j++) sc[j] = srow[j][0];
     asm volatile("" ::: "memory");
-    fetch(1u, 1u);
     uint32_t slot = 0u;
     /* stage s from `slot`; next: the codes of s + 1, refilled with s + 3 */
     auto stage = [&](uint32_t s, u32x4_t &next, auto Odd) {
         constexpr bool odd = decltype(Odd)::value;
-        /* younger than stage s's tokens: those of s + 1, a code load and four
-         * scales at least */
+        /* This wave's loads of stage s are done before the barrier, behind
+         * which its neighbours read them. Issued after those four: for stage
+         * 0 fetch(1), the codes of 2 and four scales (9); for stage 1 these
+         * five, fetch(2) and the codes of 3 (10); from stage 2 on fetch(s + 1),
+         * the codes of s + 1 and s + 2 and, at the odd stage of the two, four
+         * scales (10). */
         wait_vm<9>();
         wait_lgkm<0>(); /* this wave's code writes */
         asm volatile("" ::: "memory");
