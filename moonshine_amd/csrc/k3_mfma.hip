@@ -44,8 +44,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kTileRows[kTileClasses] = {16u, 64u, 96u, 128u};
 
-__device__ __forceinline__ float bf16r(float v) { return bf16_to_f32(f32_to_bf16(v)); }
-
 /* ---------------------------------------------------------------------- */
 /* activation split                                                        */
 /* ---------------------------------------------------------------------- */
@@ -743,19 +741,48 @@ struct GateUpArgs {
     float beta, lb;
 };
 
-/* The epilogue's sigmoid and tanh: the deterministic forms' formulas with the
- * hardware exp2 and reciprocal (each within 1 ulp) for the exponential and the
- * divisions, and no branches. This path's two-term split already carries
- * ~2^-16 relative error, and the activation is rounded to bf16 first. The
- * deterministic SiTU (two branching tanh, three divisions) took a third of
- * the K3-native gate/up launch: 2048 tokens 2.85 -> 2.38 ms (the
- * three larger token classes). Against 64-bit results the layer's error stays
- * where it was (96..1500 tokens: 4.354e-3 of the norm before and after). */
+/* SwiGLU's sigmoid on the hardware exp2 and reciprocal (instructions within 1
+ * ulp each): the path's two-term split already carries ~2^-16 relative error,
+ * and the activation is rounded to bf16 first. */
 __device__ __forceinline__ float hw_sigmoid(float x) {
     const float e = __builtin_amdgcn_exp2f(__fmul_rn(x, -1.44269502162933349609375f));
     return __builtin_amdgcn_rcpf(__fadd_rn(1.0f, e));
 }
-__device__ __forceinline__ float hw_tanh(float y) {
+
+/*
+ * SiTU with gated_act's bits, without its branches: the same tanh, sigmoid and
+ * quotients, with both sides of tanh computed and selected, and each IEEE
+ * division replaced by a hardware reciprocal and one step on the exact
+ * residual, which rounds correctly over the ranges used. Checked on the part:
+ * the reciprocal against the division over every mantissa, tanh against
+ * det_tanhf over every float, and the whole against gated_act over every pair
+ * of bf16 values for nine (beta, lb). gated_act itself (two branching tanh, five
+ * divisions) took a third of the K3-native gate/up launch; the hardware exp2
+ * with products by 1 / beta is shorter still but up to 29 ulp off. us, gated_act
+ * -> here (hardware exp2): K3-native layer, 2048 tokens 6182 -> 5380 (5250, the
+ * projections' tiles in both), its expert stage alone, 4096 tokens 6080 -> 5570
+ * (5410); 1024 x 1024, 40 experts, 8192 tokens 793 -> 640 (585).
+ */
+__device__ __forceinline__ float rcp_rn(float d) { /* 1 / d, 2^-125 <= d <= 2^125 */
+    const float y = __builtin_amdgcn_rcpf(d);
+    return fmaf(fmaf(-d, y, 1.0f), y, y);
+}
+/* 2^-shift det_expf(x) where that is a normal number and |x| <= 104 */
+__device__ __forceinline__ float exp_normal(float x, int shift) {
+    const float n = rintf(__fmul_rn(x, 1.44269502162933349609375f));
+    float r = fmaf(-n, 0.693145751953125f, x);
+    r = fmaf(-n, 1.428606765330187045037746429443359375e-6f, r);
+    float p = 1.9841270113736391067504882812e-4f;
+    p = fmaf(p, r, 1.3888889225199818611145019531e-3f);
+    p = fmaf(p, r, 8.3333337679505348205566406250e-3f);
+    p = fmaf(p, r, 4.1666667908430099487304687500e-2f);
+    p = fmaf(p, r, 1.6666667163372039794921875000e-1f);
+    p = fmaf(p, r, 0.5f);
+    p = fmaf(p, r, 1.0f);
+    p = fmaf(p, r, 1.0f);
+    return __builtin_amdgcn_ldexpf(p, (int)n - shift);
+}
+__device__ __forceinline__ float situ_tanh(float y) {
     const float a = fabsf(y), z = __fmul_rn(a, a);
     float p = -1.4558343870513183e-3f;
     p = fmaf(p, z, 3.5921280365724811e-3f);
@@ -765,9 +792,48 @@ __device__ __forceinline__ float hw_tanh(float y) {
     p = fmaf(p, z, 1.3333333333333333e-1f);
     p = fmaf(p, z, -3.3333333333333333e-1f);
     const float lo = fmaf(__fmul_rn(a, z), p, a);
-    const float e = __builtin_amdgcn_exp2f(__fmul_rn(a, 2.8853900432586669921875f));
-    const float hi = fmaf(-2.0f, __builtin_amdgcn_rcpf(__fadd_rn(e, 1.0f)), 1.0f);
-    return copysignf(a < 0.5f ? lo : hi, y); /* NaN takes hi and stays NaN */
+    const float c = a >= 9.1f ? 9.1f : a; /* 1 from there on; NaN stays */
+    const float hi = fmaf(-2.0f, rcp_rn(__fadd_rn(exp_normal(__fadd_rn(c, c), 0), 1.0f)), 1.0f);
+    return copysignf(a < 0.5f ? lo : hi, y);
+}
+/* det_sigmoid of a bf16 value: below -80 the 1 of 1 + exp(-x) is lost and the
+ * reciprocal is taken 2^64 up, from -88.7 on exp(-x) overflows */
+__device__ __forceinline__ float situ_sigmoid(float x) {
+    const bool low = x < -80.0f;
+    const float t = x > 20.0f ? -20.0f : x < -88.72283935546875f ? 89.0f : -x;
+    const float e = exp_normal(t, low ? 64 : 0);
+    const float s = __builtin_amdgcn_ldexpf(rcp_rn(__fadd_rn(low ? 0.0f : 1.0f, e)), low ? -64 : 0);
+    return x < -88.72283935546875f ? 0.0f : s;
+}
+/* v / beta; inv = 1 / beta rounded. The step is exact for 2^-100 <= |v| <
+ * 2^100 and 2^-20 <= beta <= 2^20 (else limit is 0 and no v is in range). */
+struct SituDiv {
+    float beta, inv;
+    uint32_t limit;
+    __device__ __forceinline__ explicit SituDiv(float b)
+        : beta(b), inv(__fdiv_rn(1.0f, b)),
+          limit(b >= 9.5367431640625e-7f && b <= 1048576.0f ? 0x64000000u : 0u) {}
+    __device__ __forceinline__ bool in_range(float v) const {
+        return (__float_as_uint(v) & 0x7fffffffu) - 0x0d800000u < limit;
+    }
+    __device__ __forceinline__ float operator()(float v) const {
+        const float q = __fmul_rn(v, inv);
+        return fmaf(fmaf(-q, beta, v), inv, q);
+    }
+};
+/* bf16 of SiTU beta tanh(g / beta) sigmoid(g) lb tanh(u / lb), two values */
+__device__ __forceinline__ float2 situ2(float2 g, float2 u, const SituDiv &gd, const SituDiv &ud) {
+    float2 y = make_float2(gd(g.x), gd(g.y)), z = make_float2(ud(u.x), ud(u.y));
+    const bool fits = gd.in_range(g.x) & gd.in_range(g.y) & ud.in_range(u.x) & ud.in_range(u.y);
+    if (__builtin_expect(__any(!fits), 0)) { /* the wave together: the same quotients in range */
+        y = make_float2(__fdiv_rn(g.x, gd.beta), __fdiv_rn(g.y, gd.beta));
+        z = make_float2(__fdiv_rn(u.x, ud.beta), __fdiv_rn(u.y, ud.beta));
+    }
+    auto one = [&](float gv, float yg, float zu) {
+        const float bg = __fmul_rn(gd.beta, situ_tanh(yg)), bu = __fmul_rn(ud.beta, situ_tanh(zu));
+        return __fmul_rn(__fmul_rn(bg, situ_sigmoid(gv)), bu);
+    };
+    return bf16r2(one(g.x, y.x, z.x), one(g.y, y.y, z.y));
 }
 
 /*
@@ -784,9 +850,7 @@ __device__ __forceinline__ void gateup_epilogue(const f32x4 (&acc)[C::WM][C::WN]
     constexpr int G = C::WN / 2, LB = 32 / G;
     static_assert(G == 2 || G == 4, "two or four columns per lane");
     const uint32_t F = A.F;
-    /* finite also for a denormal divisor: 0 / beta stays 0 */
-    const float inv_beta = fminf(__fdiv_rn(1.0f, A.beta), 3.4028234663852886e38f);
-    const float inv_lb = fminf(__fdiv_rn(1.0f, A.lb), 3.4028234663852886e38f);
+    const SituDiv gate_div(A.beta), up_div(A.lb);
     /* template loops: the rows must unroll fully (acc indices constant)
      * even where the activation's body exceeds the unroller's budget */
     static_for<C::WM * 4>([&](auto IR) {
@@ -808,17 +872,11 @@ __device__ __forceinline__ void gateup_epilogue(const f32x4 (&acc)[C::WM][C::WN]
                 v[j + 1] = hh.y;
             }
         } else {
-            /* SiTU beta tanh(g / beta) sigmoid(g) lb tanh(u / lb) */
-            auto situ = [&](float gv, float uv) {
-                const float bg = __fmul_rn(A.beta, hw_tanh(__fmul_rn(gv, inv_beta)));
-                const float bu = __fmul_rn(A.lb, hw_tanh(__fmul_rn(uv, inv_lb)));
-                return __fmul_rn(__fmul_rn(bg, hw_sigmoid(gv)), bu);
-            };
 #pragma unroll
             for (int j = 0; j < G; j += 2) {
                 const float2 gg = bf16r2(acc[i][j][r], acc[i][j + 1][r]);
                 const float2 uu = bf16r2(acc[i][G + j][r], acc[i][G + j + 1][r]);
-                const float2 hh = bf16r2(situ(gg.x, uu.x), situ(gg.y, uu.y));
+                const float2 hh = situ2(gg, uu, gate_div, up_div);
                 v[j] = hh.x;
                 v[j + 1] = hh.y;
                 __builtin_amdgcn_sched_barrier(0);

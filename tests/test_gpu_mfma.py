@@ -363,3 +363,56 @@ def test_k3_shape_mixed_alignment_bitexact(cuda):
     np.testing.assert_array_equal(ids_m, ids_a)
     np.testing.assert_array_equal(w_m, w_a)
     np.testing.assert_array_equal(got, ref)
+
+
+@pytest.mark.parametrize("beta,lb", [(4.0, 25.0), (1.0, 1.0)])
+def test_situ_epilogue_bits(cuda, beta, lb):
+    """The SiTU epilogue of every tile class against the oracle's SiTU, bit for
+    bit, over about a million (gate, up) pairs. The layer makes the pairs exact:
+    a token has v and w in its first two columns, gate row f reads v and up row
+    f reads w, each times a power of two of its 32-row block, and the down
+    matrix is the identity. v and w are within 2^5 of each other and a block's
+    activations equal, so the two-term split carries both exactly; activations
+    under 2^-100 (gates below -64) may be cut by its smallest scale."""
+    from types import SimpleNamespace
+    H = F = 512
+    counts = [65535 - 96 - 64 - 16, 96, 64, 16]  # 128-, 96-, 64- and 16-row tiles
+    T, E = sum(counts), len(counts)
+    rng = np.random.default_rng(int(beta))
+    block = np.arange(F) // 32
+    sign = np.where(block % 3 == 2, 8, 0)         # the e2m1 sign bit
+    gate, up = np.zeros((F, H), np.uint8), np.zeros((F, H), np.uint8)
+    gate[:, 0] = 2 | sign                           # +-1.0
+    up[:, 1] = 2 | np.where(block % 2 == 1, 8, 0)
+    down = np.zeros((H, F), np.uint8)
+    np.fill_diagonal(down, 2)
+    ge, ue = block - 9, (5 * block) % 13 - 7        # gates of 2^-9 .. 2^7, ups of 2^-8 .. 2^7
+    tensors = []
+    for codes, exp in ((gate, ge), (down, np.zeros(H, int)), (up, ue)):
+        tensors.append(codes[:, 0::2] | (codes[:, 1::2] << 4))
+        tensors.append(np.repeat((127 + exp).astype(np.uint8)[:, None], codes.shape[1] // 32, 1))
+    dev = [torch.from_numpy(np.ascontiguousarray(t)).to(cuda) for t in tensors]
+    table = torch.tensor([[t.data_ptr() for t in dev]] * E, dtype=torch.int64, device=cuda)
+    cfg = dataclasses.replace(CONFIGS[0], name="situ", tokens=T, hidden=H, ffn=F, experts=E,
+                              top_k=1, activation=0, beta=beta, linear_beta=lb)
+    moe = L.RoutedMoE(cfg, table, None, SimpleNamespace(table=table))
+    pairs = (rng.uniform(1.0, 2.0, (T, 2)) * rng.choice([-1.0, 1.0], (T, 2)) *
+             [1.0, 0.5]).astype(np.float32)
+    x = np.zeros((T, H), np.uint16)
+    x[:, :2] = f32_to_bf16_bits(pairs)
+    ids = np.repeat(np.arange(E, dtype=np.int32), counts)[:, None]
+    out = moe.experts_only(L.bf16_tensor(x, cuda), torch.from_numpy(ids).to(cuda),
+                           torch.ones((T, 1), dtype=torch.float32, device=cuda), precision=MFMA)
+    torch.cuda.synchronize()
+    got = L.bf16_bits(out)[:, ::32]
+    first = np.arange(0, F, 32)
+    v, w = (bf16_bits_to_f32(x[:, c])[:, None] for c in (0, 1))
+    g = v * np.ldexp(1.0, ge[first]) * np.where(sign[first], -1.0, 1.0)
+    u = w * np.ldexp(1.0, ue[first]) * np.where(block[first] % 2 == 1, -1.0, 1.0)
+    want = O.situ(f32_to_bf16_bits(g.astype(np.float32)), f32_to_bf16_bits(u.astype(np.float32)),
+                  beta, lb)
+    big = np.abs(bf16_bits_to_f32(want)) >= 2.0 ** -100
+    assert big.mean() > 0.9
+    bad = big & (got != want)
+    assert not bad.any(), f"{bad.sum()} of {bad.size} differ, first at {np.argwhere(bad)[0]}"
+    assert np.abs(bf16_bits_to_f32(got)[~big]).max(initial=0.0) <= 2.0 ** -99
