@@ -31,6 +31,7 @@
  */
 #include "k3_device.h"
 #include "k3_exact.h"
+#include "k3_exact_rule.h"
 #include "k3_lds.h"
 
 #include <hip/hip_runtime.h>
@@ -729,11 +730,8 @@ __device__ __forceinline__ bool dense_tile(const DenseArgs &A, uint32_t wk, uint
     return true;
 }
 
-/* blocks of a CU: the 16-token tiles of 64 rows take all its registers */
-constexpr int dense_blocks(int RB, int NT) { return RB == 64 && NT > 2 ? 1 : 2; }
-
 template <class Fmt, int NT, int RB>
-__global__ __launch_bounds__(512, 2 * dense_blocks(RB, NT)) void exact_dense_kernel(DenseArgs A) {
+__global__ __launch_bounds__(512, RB == 64 && NT > 2 ? 2 : 4) void exact_dense_kernel(DenseArgs A) {
     constexpr int SB = RB == 64 && NT <= 2 ? 256 : 512;
     __shared__ __attribute__((aligned(16))) uint8_t smem[RB * (kRing * SB + 2 * kScaleGroups)];
     using C = Core<Fmt, NT, 0, SB, RB>;
@@ -764,30 +762,19 @@ __global__ __launch_bounds__(512, 2 * dense_blocks(RB, NT)) void exact_dense_ker
     }
 }
 
-constexpr uint32_t kCus = 256; /* persistent grids: blocks of a CU times this */
-
-/* 16-row tiles where 64-row ones would leave CUs idle: a tile's time is the
- * floor then, and the smaller tile's is a third. Measured, 64-row against
- * 16-row: MXFP4 3072 x 3584 at 32 tokens (96 works of 64 rows x 16 tokens)
- * 23.9 against 19.2 us, at 48 (144) 24.0 against 25.2; 2048 x 7168 at 64
- * (128) 41.8 against 33.0, at 96 (192) 42.4 against 44.1. Up to 8 tokens the
- * 64-row tile is itself shorter: Q8-128 6144 x 7168 at 8 tokens (96) 32.6
- * against 35.3, 3584 x 7168 (56) 32.0 against 23.7. */
-constexpr uint64_t few_works(uint32_t tokens) { return tokens <= 8u ? 64u : 128u; }
-
+/* persistent grids: blocks of a CU times the CUs */
 uint32_t grid_of(uint64_t works, uint32_t per_cu) {
     return (uint32_t)(works < per_cu * kCus ? works : per_cu * kCus);
 }
 
 template <class Fmt, int NT, int RB>
-bool launch_dense_tiles(DenseArgs A, hipStream_t st) {
-    const uint32_t TT = NT * 256 / RB;
-    A.token_tiles = (A.tokens + TT - 1u) / TT;
+bool launch_dense_tiles(DenseArgs A, const DenseForm &f, hipStream_t st) {
+    A.token_tiles = (A.tokens + f.tokens() - 1u) / f.tokens();
     const uint64_t works = (uint64_t)((A.rows + RB - 1u) / RB) * A.token_tiles;
     if (works > 0xffff0000ull) return false;
     A.works = (uint32_t)works;
     hipLaunchKernelGGL(HIP_KERNEL_NAME(exact_dense_kernel<Fmt, NT, RB>),
-                       dim3(grid_of(works, dense_blocks(RB, NT))), dim3(64 * W), 0, st, A);
+                       dim3(grid_of(works, f.per_cu)), dim3(64 * W), 0, st, A);
     return hipGetLastError() == hipSuccess;
 }
 
@@ -796,11 +783,11 @@ bool launch_dense(uint16_t *out, const void *w, const void *s, const void *x, ui
                   uint32_t rows, uint32_t cols, hipStream_t st) {
     const DenseArgs A{out, (const uint8_t *)w, (const uint8_t *)s, (const uint16_t *)x, tokens,
                       rows, cols, 0u, 0u};
-    const uint64_t works = (uint64_t)((rows + kRows - 1u) / kRows) * ((tokens + 15u) / 16u);
-    if (works <= few_works(tokens)) return launch_dense_tiles<Fmt, 1, 16>(A, st);
-    if (tokens <= 4u) return launch_dense_tiles<Fmt, 1, 64>(A, st);
-    if (tokens <= 8u) return launch_dense_tiles<Fmt, 2, 64>(A, st);
-    return launch_dense_tiles<Fmt, 4, 64>(A, st);
+    const DenseForm f = dense_form(tokens, rows);
+    if (f.rows == 16u) return launch_dense_tiles<Fmt, 1, 16>(A, f, st);
+    if (f.quads == 1u) return launch_dense_tiles<Fmt, 1, 64>(A, f, st);
+    if (f.quads == 2u) return launch_dense_tiles<Fmt, 2, 64>(A, f, st);
+    return launch_dense_tiles<Fmt, 4, 64>(A, f, st);
 }
 
 /* The light and the heavy tiles' launches (a token has an expert at most

@@ -19,6 +19,7 @@
  */
 #include "k3_device.h"
 #include "k3_exact.h"
+#include "k3_exact_rule.h"
 #include "k3_internal.h"
 #include "k3_topk.h"
 #include "../../include/k3_rocm_ops.h"
@@ -488,7 +489,7 @@ __device__ __forceinline__ uint4 load_group(const uint8_t *p, uint32_t align16) 
 
 /* One wave per weight row, TT tokens: all of a row's loads in flight at once,
  * so a small product costs one memory round trip; its vector arithmetic grows
- * with the tokens (rows_form). */
+ * with the tokens (dense_rows_form). */
 template <int TT>
 __global__ __launch_bounds__(256) void mxfp4_rows_kernel(
         uint16_t *__restrict__ out, const uint8_t *__restrict__ packed,
@@ -1066,15 +1067,6 @@ extern "C" bool k3_rocm_swiglu_bf16(void *output, const void *gate, const void *
     return hipGetLastError() == hipSuccess;
 }
 
-/* Products that stay on the one-wave-per-row kernels: one vector (bound by
- * memory), and up to 16384 outputs. Measured either side of it, rows against
- * matrix kernels: MXFP4 3072 x 3584 at 5 tokens 9.9 against 11.7 us and at 8
- * 13.8 against 12.0; 512 x 2048 at 32 6.7 against 8.4 and at 48 10.0 against
- * 8.4; Q8-128 6144 x 7168 at 2 18.8 against 26.6 and at 4 29.2 against 25.9. */
-static bool rows_form(uint32_t tokens, uint32_t rows) {
-    return tokens == 1u || (uint64_t)tokens * rows <= 16384u;
-}
-
 /* the tile is the reference's; results do not depend on it */
 static bool batch_tile_ok(uint32_t tile) { return tile == 16u || tile == 32u || tile == 64u; }
 
@@ -1096,7 +1088,7 @@ extern "C" bool k3_rocm_mxfp4_gemm_bf16(void *output, const void *packed, const 
         ((uintptr_t)packed % 8u) != 0u || ((uintptr_t)input % 16u) != 0u)
         return false;
     const hipStream_t s = (hipStream_t)stream;
-    if (!rows_form(vector_count, rows))
+    if (!k3::dense_rows_form(vector_count, rows, columns, false))
         return k3::launch_exact_mxfp4((uint16_t *)output, packed, scales, input, vector_count,
                                       rows, columns, s);
     if (vector_count == 1u)
@@ -1316,7 +1308,7 @@ extern "C" bool k3_rocm_q8_128_gemm_bf16(void *output, const void *quantized, co
                                          uint32_t columns, void *stream) {
     if (!q8_args_ok(output, quantized, scales, input, vector_count, rows, columns)) return false;
     const hipStream_t s = (hipStream_t)stream;
-    if (!rows_form(vector_count, rows))
+    if (!k3::dense_rows_form(vector_count, rows, columns, true))
         return k3::launch_exact_q8((uint16_t *)output, quantized, scales, input, vector_count,
                                    rows, columns, s);
     if (vector_count == 1u) {
