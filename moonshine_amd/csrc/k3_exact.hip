@@ -791,16 +791,17 @@ bool launch_dense(uint16_t *out, const void *w, const void *s, const void *x, ui
 }
 
 /* The light and the heavy tiles' launches (a token has an expert at most
- * once, so few tokens make no heavy tiles); a list of experts runs on the
- * heavy kernel over a grid of its own, the list being empty as a rule. */
-constexpr uint32_t kListBlocks = 64;
-
+ * once, so few tokens make no heavy tiles). A list of experts (tensors that the
+ * scaled-MFMA tiles cannot take; none as a rule) runs on the heavy kernel, one
+ * block a CU: an empty list costs no more than on 64 blocks, on which a layer
+ * of 128 such experts (3584 / 2048) took 762 us for 9 tokens and 2240 for 64
+ * against 273 and 663 here. */
 template <class Args>
 bool launch_grouped(const Args &A, uint32_t ncol, hipStream_t st) {
     const ExactGroup &g = A.g;
     const dim3 block(64 * W);
     if (g.list) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(exact_tiles_run_kernel<true, Args>), dim3(kListBlocks),
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(exact_tiles_run_kernel<true, Args>), dim3(kCus),
                            block, 0, st, A);
         return hipGetLastError() == hipSuccess;
     }
