@@ -245,9 +245,10 @@ def test_proj_mfma_ragged_vs_row_kernels(cuda, q8, T, rows, cols):
 
 
 @pytest.mark.parametrize("T,rows,cols", [
-    (65, 129, 128), (1, 65, 3584), (300, 577, 768), (129, 200, 896),      # 64 x 64 tiles
-    (1000, 1030, 128), (961, 1025, 640),                                  # 64 x 128
-    (2000, 1090, 128), (1921, 1153, 512),                                 # 128 x 128
+    (65, 129, 128), (1000, 1030, 128), (2000, 1090, 128),                 # one scale block
+    (65, 129, 256), (1, 65, 3584), (300, 577, 768), (129, 200, 896),      # 64 x 64 tiles
+    (1000, 1030, 256), (961, 1025, 640),                                  # 64 x 128
+    (2000, 1090, 256), (1921, 1153, 512),                                 # 128 x 128
     (32769, 128, 128), (1025, 4100, 256), (2055, 2100, 384), (1279, 3201, 3584)])  # 256 x 128
 def test_proj_mfma_q8_tiles(cuda, T, rows, cols):
     """Every tile of the Q8 projections where its rounds make it the choice:
@@ -256,8 +257,8 @@ def test_proj_mfma_q8_tiles(cuda, T, rows, cols):
     test_proj_mfma_ragged_vs_row_kernels(cuda, True, T, rows, cols)
 
 
-@pytest.mark.parametrize("T,rows,cols", [(65, 129, 384), (961, 1025, 128), (1921, 1153, 128),
-                                         (1025, 4100, 256)])
+@pytest.mark.parametrize("T,rows,cols", [(65, 129, 384), (961, 1025, 128), (961, 1025, 256),
+                                         (1921, 1153, 256), (1025, 4100, 256)])
 def test_proj_mfma_q8_codes_at_8_mod_16(cuda, T, rows, cols):
     """Each tile with the codes at 8 mod 16: the bits of the aligned call."""
     import ctypes
@@ -276,3 +277,24 @@ def test_proj_mfma_q8_codes_at_8_mod_16(cuda, T, rows, cols):
         assert lib().k3_moe_proj_mfma_bf16(P(o), P(w), P(s), P(x), T, rows, cols, True, st)
     torch.cuda.synchronize()
     assert torch.equal(out[0].view(torch.int16), out[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("T,rows,cols", [(1000, 1030, 128), (1000, 1030, 640), (2000, 1090, 512),
+                                         (32769, 128, 128), (1025, 4100, 1152)])
+def test_proj_mfma_q8_tiles_same_bits(cuda, T, rows, cols):
+    """Every tile sums in the same order: the first tokens and rows of a call
+    have the bits of a call of their own, which takes 64 x 64 tiles."""
+    import ctypes
+    from moonshine_amd._lib import lib
+    g = torch.Generator().manual_seed(T + cols)
+    x = torch.randn((T, cols), generator=g).to(torch.bfloat16).to(cuda)
+    q = torch.randint(-127, 128, (rows, cols), generator=g, dtype=torch.int8).to(cuda)
+    s = torch.rand((rows, cols // 128), generator=g).to(cuda)
+    P = lambda t: ctypes.c_void_p(t.data_ptr())
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    whole = torch.zeros((T, rows), dtype=torch.bfloat16, device=cuda)
+    part = torch.zeros((300, 128), dtype=torch.bfloat16, device=cuda)
+    assert lib().k3_moe_proj_mfma_bf16(P(whole), P(q), P(s), P(x), T, rows, cols, True, st)
+    assert lib().k3_moe_proj_mfma_bf16(P(part), P(q), P(s), P(x), 300, 128, cols, True, st)
+    torch.cuda.synchronize()
+    assert torch.equal(whole[:300, :128].contiguous().view(torch.int16), part.view(torch.int16))
