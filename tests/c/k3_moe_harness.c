@@ -12,7 +12,7 @@
  * residual; routes on the device, one synchronisation at the end, no host
  * round trip between layers -- the sync at k3_engine.cu:1569 is not
  * needed), and the prefill router entry point (k3_moe_router_bf16) on a
- * 40-token batch. Exit status 0 = match.
+ * 96-token batch. Exit status 0 = match.
  */
 #include <hip/hip_runtime_api.h>
 
@@ -185,9 +185,9 @@ int main(void) {
     hipHostFree(layer_w);
 
     /* the prefill router entry point on a token batch (the certified MFMA
-     * form from 32 tokens on) against the oracle's logits and top-k */
+     * form from 80 tokens on) against the oracle's logits and top-k */
     {
-        const uint32_t T = 40u;
+        const uint32_t T = 96u;
         uint16_t *xb = bf16_array((size_t)T * H, 1.3f);
         void *d_xb = dev_copy(xb, 2 * (size_t)T * H);
         const size_t rs = k3_moe_router_scratch_bytes(T, E);
@@ -198,8 +198,8 @@ int main(void) {
         CHECK(hipMalloc(&d_rw, 4 * T * K) == hipSuccess);
         CHECK(k3_moe_router_bf16(d_rids, d_rw, d_xb, d_w, d_b, T, E, H, K, 2.5f, d_scratch, rs,
                                  NULL));
-        uint32_t got_ids[40 * K], want_ids[40 * K];
-        float got_w[40 * K], want_w[40 * K];
+        uint32_t got_ids[96 * K], want_ids[96 * K];
+        float got_w[96 * K], want_w[96 * K];
         float *logits = malloc(4 * (size_t)T * E);
         CHECK(hipMemcpy(got_ids, d_rids, sizeof got_ids, hipMemcpyDeviceToHost) == hipSuccess);
         CHECK(hipMemcpy(got_w, d_rw, sizeof got_w, hipMemcpyDeviceToHost) == hipSuccess);

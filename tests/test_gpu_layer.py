@@ -442,7 +442,7 @@ class MappedHost:
         self.hip.hipHostFree(self.host)
 
 
-@pytest.mark.parametrize("T", [1, 5, 40])  # 40: the certified MFMA router
+@pytest.mark.parametrize("T", [1, 5, 96])  # 96: the certified MFMA router
 def test_routes_into_mapped_host_memory(cuda, T):
     """The layer's optional route copies written straight into host-mapped
     memory, as the reference engine reads them."""
@@ -562,4 +562,4 @@ def test_c_harness():
     assert r.returncode == 0, r.stdout + r.stderr
     assert r.stdout.count("output match, ids match, weights match") == 2
     assert "4-layer decode chain (one stream, one sync) match" in r.stdout
-    assert "router entry point, 40 tokens: ids and weights match" in r.stdout
+    assert "router entry point, 96 tokens: ids and weights match" in r.stdout

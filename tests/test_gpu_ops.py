@@ -163,9 +163,8 @@ def test_mxfp4_extreme_scales(cuda, T):
 
 
 @pytest.mark.parametrize("T,E,H", [(1, 896, 7168), (3, 64, 2048), (17, 896, 7168), (4, 100, 1001),
-                                   # blocked-GEMM path (T >= 128): ragged token/row tiles,
-                                   # a partial last K step (65 chunks), XCD grouping with a
-                                   # remainder (9 row tiles) and without (7 row tiles)
+                                   # many tokens: ragged token and row groups, an odd count of
+                                   # chunks (65: one parity has more), a single chunk
                                    (300, 896, 7168), (129, 100, 520), (1000, 137, 1024),
                                    (128, 16, 8)])
 def test_router_logits_bitexact(cuda, T, E, H):

@@ -3,6 +3,8 @@ exact prefill router pair k3_rocm_bf16_gemm_f32 + k3_rocm_router_topk_f32_batch
 (k3_engine_prefill.inc:1448-1460): ids and weights bit-identical on every
 token, including exact ties, all-zero, huge, tiny and non-finite tokens."""
 import ctypes
+import pathlib
+import re
 
 import numpy as np
 import pytest
@@ -13,6 +15,11 @@ from moonshine_amd._lib import lib
 from moonshine_amd.synth import CONFIGS, f32_to_bf16_bits, make_inputs
 
 pytestmark = pytest.mark.gpu
+
+# from this many tokens on the router is the certified one
+CERTIFIED = int(re.search(r"kCertifiedMinTokens = (\d+);", (
+    pathlib.Path(__file__).resolve().parents[1] / "moonshine_amd" / "csrc" /
+    "k3_internal.h").read_text()).group(1))
 
 
 def dev(a, cuda):
@@ -54,7 +61,7 @@ def check(w_bits, bias, x_bits, k, scale, cuda, bound_rows=None):
     got_ids, got_w, approx = certified_routes(w, b, x, T, E, H, k, scale, cuda)
     np.testing.assert_array_equal(got_ids, want_ids)
     np.testing.assert_array_equal(got_w.view(np.uint32), want_w.view(np.uint32))
-    if bound_rows is not None and T >= 32:
+    if bound_rows is not None and T >= CERTIFIED:
         # the MFMA logits sit inside the error bound the candidates rely on:
         # |a - l| <= (H / 32 + 270) u ||w_e|| ||x_t||, u = 2^-24 (both sums'
         # rounding)
@@ -80,8 +87,10 @@ def test_certified_router_k3_prefill(cuda):
 
 
 @pytest.mark.parametrize("T,E,H,k", [(128, 64, 512, 4), (300, 200, 1024, 8), (517, 896, 7168, 16),
-                                     (1000, 1024, 8192, 32), (130, 40, 64, 1), (33, 896, 7168, 16),
-                                     (64, 256, 2048, 8), (31, 64, 512, 4), (129, 896, 7168, 16),
+                                     (1000, 1024, 8192, 32), (130, 40, 64, 1),
+                                     (CERTIFIED, 896, 7168, 16), (CERTIFIED + 1, 256, 2048, 8),
+                                     (CERTIFIED - 1, 896, 7168, 16), (31, 64, 512, 4),
+                                     (CERTIFIED + 16, 64, 512, 4), (129, 896, 7168, 16),
                                      (257, 1000, 1024, 8), (1024, 896, 7168, 16),
                                      (1500, 300, 1024, 8), (2048, 64, 512, 32)])
 def test_certified_router_shapes(cuda, T, E, H, k):
