@@ -48,7 +48,8 @@ bool launch_exact_gateup(const ExactGroup &g, uint16_t *act, const uint16_t *x, 
 bool launch_exact_down(const ExactGroup &g, uint16_t *y, const uint16_t *act, hipStream_t st);
 
 /* out [tokens, rows] = w [rows, cols] . x [tokens, cols]; x 16-byte aligned.
- * MXFP4: cols % 32 == 0; Q8-128 (int8 codes, f32 scales): cols % 128 == 0. */
+ * MXFP4: cols % 32 == 0; Q8-128 (int8 codes, f32 scales): cols % 128 == 0;
+ * which products come here: dense_rows_form (k3_exact_rule.h). */
 bool launch_exact_mxfp4(uint16_t *out, const void *packed, const void *scales, const void *x,
                         uint32_t tokens, uint32_t rows, uint32_t cols, hipStream_t st);
 bool launch_exact_q8(uint16_t *out, const void *codes, const void *scales, const void *x,

@@ -70,8 +70,9 @@ bool static_ok(const k3_moe_static_weight &w, uint32_t rows, uint32_t cols) {
 
 /* out [T, rows] = w . in [T, columns] with the static weight's own kernel */
 /* Token batches (T >= 32) under the MXFP8 precisions: bf16 MFMA with the
- * exact products and fp32 sums (k3_proj.hip); otherwise the exact rows
- * kernels of the reference entry points. */
+ * exact products and fp32 sums (k3_proj.hip); otherwise the reference entry
+ * points' exact kernels (Q8-128 batches on the fp32 matrix units from the
+ * sizes of dense_rows_form on). */
 constexpr uint32_t kProjMfmaMinTokens = 32;
 
 bool project(const k3_moe_static_weight &w, void *out, const void *in, uint32_t T,

@@ -1,8 +1,8 @@
 /*
  * Static projections of a token batch on bf16 MFMA, for the MXFP8
- * precisions of the K3-native block (the exact precision keeps the VALU
- * rows kernels of k3_rocm_q8_128_gemm_bf16 / k3_rocm_bf16_gemm_bf16,
- * k3_rocm_ops.cu:663-835, 1694-2038, and their bits).
+ * precisions of the K3-native block (the exact precision runs
+ * k3_rocm_q8_128_gemm_bf16 / k3_rocm_bf16_gemm_bf16, k3_rocm_ops.cu:663-835,
+ * 1694-2038, in their w64 order).
  *
  *   out[t, r] = bf16(sum_b s[r, b] * sum_{k in block b} q[r, k] x[t, k])   Q8-128
  *   out[t, r] = bf16(sum_k w[r, k] x[t, k])                                bf16
