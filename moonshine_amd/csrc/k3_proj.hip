@@ -184,7 +184,8 @@ __global__ __launch_bounds__(512) void proj_mfma_kernel(ProjArgs P) {
  * ahead, converted and written one ahead, after the stage's MFMAs. LDS
  * accesses and their waits are explicit: the compiler would drain the loads
  * in flight before each. 2048 tokens, before -> after, us: 6144 x 7168
- * 308 -> 251, 7168 x 3584 201 -> 127; 8192 tokens 1231 -> 805, 724 -> 468.
+ * 308 -> 251 (226 on the 128 x 128 tiles below, which q8_tile gives that size),
+ * 7168 x 3584 201 -> 127; 8192 tokens 1231 -> 805, 724 -> 468.
  */
 constexpr uint32_t kWT = 256, kWN = 128;              /* block tile */
 constexpr uint32_t kWA = kWT * 128u, kWB = kWN * 128u; /* bytes of a stage */
