@@ -25,9 +25,9 @@
  * rows costs 8.1 cycles per MFMA plus its conversions and sums. Per group and
  * SIMD, operands in registers: one quad of tokens 195 ns, two 300, four 545
  * (124 TFLOP/s; Q8-128 614). Measured on the vector units before and here:
- * K3 layer of 333 tokens 19.6 -> 8.0 ms, of 5 tokens 732 -> 403 us (both
- * with the router's logits, 28 -> 10 us at 5); one expert's 77 rows 326 -> 93 us; Q8-128 6144 x 7168 at 300 tokens 1.50 ->
- * 0.39 ms.
+ * K3 layer of 333 tokens 19.6 -> 8.0 ms, of 5 tokens 732 -> 403 us (both with
+ * the router's logits, 28 -> 10 us at 5); one expert's 77 rows 326 -> 93 us;
+ * Q8-128 6144 x 7168 at 300 tokens 1.50 -> 0.39 ms.
  */
 #include "k3_device.h"
 #include "k3_exact.h"

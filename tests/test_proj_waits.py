@@ -1,7 +1,7 @@
-"""The waits of the 256 x 128 Q8 projection kernel (proj_wide_kernel), replayed
-on the CPU over the instructions its source compiles to: a wave may pass the
-barrier that opens stage s only when its own direct-to-LDS loads of stage s are
-done, since its neighbours read the rows it loads."""
+"""The waits of the Q8 projection kernels, replayed on the CPU over the
+instructions their source compiles to: a wave may pass the barrier that opens
+stage s only when its own direct-to-LDS loads of stage s are done, since its
+neighbours read the rows it loads."""
 import pathlib
 import re
 import shutil
@@ -10,7 +10,14 @@ import subprocess
 import pytest
 
 ROOT = pathlib.Path(__file__).resolve().parents[1]
-LOADS = 4  # direct-to-LDS loads of a wave and stage
+pytestmark = pytest.mark.skipif(
+    shutil.which("hipcc") is None and not pathlib.Path("/opt/rocm/bin/hipcc").exists(),
+    reason="needs the compiler")
+
+
+@pytest.fixture(scope="module")
+def proj(tmp_path_factory):
+    return device_assembly("csrc/k3_proj.hip", tmp_path_factory.mktemp("proj"))
 
 
 def device_assembly(source, tmp_path):
@@ -65,11 +72,31 @@ def replay(lines, barriers):
     return seen
 
 
-@pytest.mark.skipif(shutil.which("hipcc") is None and not pathlib.Path("/opt/rocm/bin/hipcc").exists(),
-                    reason="needs the compiler")
-def test_wide_stage_loads_are_done_at_its_barrier(tmp_path):
-    lines = kernel_lines(device_assembly("csrc/k3_proj.hip", tmp_path), "proj_wide_kernel")
-    for stage, (issued, flight) in enumerate(replay(lines, 8)):
-        assert issued == LOADS * (stage + 2)  # two stages ahead
-        late = [f for f in flight if f < LOADS * (stage + 1)]
-        assert not late, f"stage {stage}: loads {late} still in flight behind its barrier"
+def check(stage, need, flight):
+    late = [f for f in flight if f < need]
+    assert not late, f"stage {stage}: loads {late} still in flight behind its barrier"
+
+
+# kernel, loads of a wave and stage, stages fetched ahead of the first barrier
+@pytest.mark.parametrize("name,loads,ahead", [("proj_wide_kernel", 4, 2),
+                                              ("proj_ring_kernelILi2ELi1ELi2ELi2E", 4, 1),
+                                              ("proj_ring_kernelILi2ELi1ELi2ELi6E", 4, 5)])
+def test_stage_loads_are_done_at_its_barrier(proj, name, loads, ahead):
+    for stage, (issued, flight) in enumerate(replay(kernel_lines(proj, name), 8)):
+        assert issued == loads * (stage + ahead)
+        check(stage, loads * (stage + 1), flight)
+
+
+@pytest.mark.parametrize("name,loads,ring,phases", [("proj_ring_kernelILi2ELi2ELi2ELi4E", 5, 4, 2),
+                                                    ("proj_ring_kernelILi4ELi2ELi2ELi3E", 7, 3, 4)])
+def test_alternating_halves_wait_a_barrier_early(proj, name, loads, ring, phases):
+    """Half of the block runs one barrier behind: the loads of stage s + 1 are
+    done before the last but one of stage s's barriers."""
+    groups = {}
+    for issued, flight in replay(kernel_lines(proj, name), 2 + 6 * phases):
+        groups.setdefault(issued, []).append(flight)
+    check(0, loads, groups.pop(loads * (ring - 1))[0])
+    for stage in range(5):
+        barriers = groups.pop(loads * (ring + stage))
+        assert len(barriers) == phases
+        check(stage + 1, loads * (stage + 2), barriers[-2])
